@@ -90,6 +90,8 @@ SIGNATURES = {
                               _i32, _vp, _sz, _vp]),
     'a4g_attention_i8': (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64), _i32, _i32,
                                 _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
+    'a4g_attention_long_i8': (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64), _i32, _i32,
+                                _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     'a4g_packed_ld_f': (_i64, [_i64, _i32]),
     'a4g_pack_weights_f': (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp]),
     'a4g_dense_f': (_i32, [_vp, _i32, _i32, _i64, _vp, _i64, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _vp]),

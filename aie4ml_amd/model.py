@@ -347,14 +347,16 @@ class GPUModel:
                 self._run_attention_unfused(grp, values, heads_view=(q, k, v))
                 return
             out = torch.empty((q.shape[0], q.shape[2], nh * d), dtype=torch.int8, device=q.device)
-            ops.attention(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode,
-                          out=out.unflatten(-1, (nh, d)).permute(0, 2, 1, 3))
+            attend = ops.attention_long if ops.attention_is_long(d, int(k.shape[-2])) else ops.attention
+            attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode,
+                   out=out.unflatten(-1, (nh, d)).permute(0, 2, 1, 3))
             values[grp['out']] = out
         elif not _views_are_16_byte_aligned(values[tr0['q']], values[tr0['k']], values[tr0['v']]):
             self._run_attention_unfused(grp, values)
         else:
-            values[grp['out']] = ops.attention(values[tr0['q']], values[tr0['k']], values[tr0['v']], c1.shift, c1.rounding_mode,
-                                               sm, c3.shift, c3.rounding_mode)
+            q, k, v = values[tr0['q']], values[tr0['k']], values[tr0['v']]
+            attend = ops.attention_long if ops.attention_is_long(int(q.shape[-1]), int(k.shape[-2])) else ops.attention
+            values[grp['out']] = attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode)
 
     def _run_attention_unfused(self, grp, values, heads_view=None) -> None:
         """The members of a planned attention group one operator at a time: MatMul, Softmax, MatMul per head, then the

@@ -611,6 +611,22 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logit_shift: in
     head_dim 80 on -, unaligned views). Head dimensions 16, 48, 80, 96 and 112 run on the next wider kernel (32, 64, 128) with the pieces of a
     row that do not exist masked inside it.
     """
+    return _attention('a4g_attention_i8', q, k, v, logit_shift, logit_rounding, softmax, out_shift, out_rounding, out)
+
+
+def attention_is_long(head_dim: int, keys: int) -> bool:
+    """Whether a fused attention call of this size is attention_long()'s: more keys than attention() keeps in registers."""
+    return keys > (256 if head_dim > 64 else 512)
+
+
+def attention_long(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logit_shift: int, logit_rounding, softmax: dict,
+                   out_shift: int, out_rounding, out: Optional[torch.Tensor] = None):
+    """attention() for any number of keys up to 32768 (same arguments, same integers, one launch): the kernel walks the keys
+    of a row three times instead of keeping their logits."""
+    return _attention('a4g_attention_long_i8', q, k, v, logit_shift, logit_rounding, softmax, out_shift, out_rounding, out)
+
+
+def _attention(entry: str, q, k, v, logit_shift, logit_rounding, softmax, out_shift, out_rounding, out):
     for name, t in (('q', q), ('k', k), ('v', v)):
         _dev(t, name)
         if t.dtype != torch.int8 or t.dim() < 2 or t.dim() > 4 or t.stride(-1) != 1:
@@ -638,7 +654,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logit_shift: in
     kind = softmax.get('kind', 'exp')
     if kind not in ('exp', 'hccs'):
         raise ValueError(f"attention: unknown softmax kind {kind!r}")
-    check(_lib.load().a4g_attention_i8(_ptr(q), _ptr(k), _ptr(v), _ptr(out), batch, heads, sq, sk, d, arr, int(logit_shift),
+    check(getattr(_lib.load(), entry)(_ptr(q), _ptr(k), _ptr(v), _ptr(out), batch, heads, sq, sk, d, arr, int(logit_shift),
                                        _mode(logit_rounding), 0 if kind == 'exp' else 1, int(softmax.get('exp_kq', 1)),
                                        int(softmax.get('B', 0)), int(softmax.get('S', 0)), int(softmax.get('Dmax', 0)),
                                        int(softmax.get('inv_shift', 15)), int(bool(softmax.get('use_clb', False))),

@@ -459,8 +459,9 @@ class PlanGpuFusion(AIEPass):
                 and cfg.n_in <= self.ROWLN_MAX_K and cfg.n_out >= 384)
 
     # ---- attention -------------------------------------------------------------------------------------
-    # head dimension -> keys the fused kernel takes (16, 48, 80, 96, 112 run padded to 32, 64, 128)
-    ATTN_MAX_KEYS = {16: 512, 32: 512, 48: 512, 64: 512, 80: 256, 96: 256, 112: 256, 128: 256}
+    # what the fused kernels take: head dimensions that are multiples of 16 up to 128, up to 32768 keys
+    ATTN_MAX_DIM = 128
+    ATTN_MAX_KEYS = 32768
     ATTN_MAX_SHIFT = 24
 
     def _plan_attention(self, graph, execution, outputs):
@@ -492,7 +493,7 @@ class PlanGpuFusion(AIEPass):
             if len(q.shape) != len(k.shape) or len(k.shape) != len(v.shape) or tuple(k.shape) != tuple(v.shape) \
                     or tuple(q.shape[:-2]) != tuple(k.shape[:-2]) or len(q.shape) not in (2, 3, 4):
                 continue
-            if not 1 <= int(k.shape[-2]) <= self.ATTN_MAX_KEYS.get(int(q.shape[-1]), 0):
+            if int(q.shape[-1]) % 16 or int(q.shape[-1]) > self.ATTN_MAX_DIM or not 1 <= int(k.shape[-2]) <= self.ATTN_MAX_KEYS:
                 continue
             if c1.shift > self.ATTN_MAX_SHIFT or c3.shift > self.ATTN_MAX_SHIFT:
                 continue  # the fused kernel takes shifts up to 24, the MatMul kernels up to 31

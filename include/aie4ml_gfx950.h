@@ -311,6 +311,15 @@ A4G_API int a4g_attention_i8(const int8_t* Q, const int8_t* K, const int8_t* V, 
                      int logit_round_mode, int softmax_kind, int exp_kq, int hccs_B, int hccs_S, int hccs_Dmax,
                      int inv_shift, int use_clb, int out_shift, int out_round_mode, a4g_stream_t stream);
 
+/* The same for any number of keys: arguments, operations and results of a4g_attention_i8, up to 32768 keys for every
+ * head dimension that is a multiple of 16 up to 128. It walks the keys of a row three times instead of keeping their
+ * logits, which makes it the slower of the two where both apply; a caller takes it for what a4g_attention_i8 answers
+ * with A4G_ERR_UNSUPPORTED (more than 512 keys, 256 from head dimension 80 on). */
+A4G_API int a4g_attention_long_i8(const int8_t* Q, const int8_t* K, const int8_t* V, int8_t* O, int64_t batch, int64_t heads,
+                     int64_t sq, int64_t sk, int64_t d, const int64_t* strides, int logit_shift,
+                     int logit_round_mode, int softmax_kind, int exp_kq, int hccs_B, int hccs_S, int hccs_Dmax,
+                     int inv_shift, int use_clb, int out_shift, int out_round_mode, a4g_stream_t stream);
+
 /* ---- Floating-point compute path ------------------------------------------------------------------
  * The reference's float mode (FloatIntent tensors, passes/force_float_mode.py): bfloat16, float32 or fp8
  * e4m3 operands, float32 accumulation (acc_scalar_t = accfloat), results converted to the operand format:

@@ -241,3 +241,24 @@ def test_attention_uncovered_shapes_and_bad_parameters():
         ops.attention(q, q, q, 6, 'floor', {'kind': 'hccs', 'B': 600, 'S': 1, 'Dmax': 5}, 7, 'floor')
     with pytest.raises(ValueError, match='incompatible shapes'):
         ops.attention(q, q[:, :32], q, 6, 'floor', {'kind': 'exp', 'exp_kq': 23}, 7, 'floor')
+
+
+@pytest.mark.parametrize('d,sq,sk', [(64, 513, 513), (64, 3, 544), (64, 130, 1024), (48, 70, 600), (32, 129, 577), (16, 40, 520),
+                                     (128, 257, 257), (80, 100, 700), (128, 9, 1030), (64, 5, 1), (32, 33, 31), (64, 65, 129)])
+@pytest.mark.parametrize('mode', ['conv_even', 'symmetric_inf', 'symmetric_zero', 'floor'])
+def test_attention_long(oracle, d, sq, sk, mode):
+    """The kernel that walks the keys three times: key counts on and off its tiles, chunks and groups of tiles (and below
+    one of each), every head width, every form of the logit requantisation, both forms of the probability; rows of K
+    and V that lie in a wider tensor whose bytes around them hold extreme values."""
+    q, k, v = qkv(d + sq + sk, (2, 2, sq, d), (2, 2, sk, d), sigma=30.0)
+    k[0, 0], v[1, 1] = -np.abs(k[0, 0]), 127  # a head whose logits lean one way; a head whose sums are as large as they get
+    wide = [np.full((2, 2, sk + 3, d + 16), 127, np.int8) for _ in range(2)]
+    wide[0][:, :, :sk, :d], wide[1][:, :, :sk, :d] = k, v
+    wk, wv = (dev(t)[:, :, :sk, :d] for t in wide)
+    B = min(255, 32767 // sk)
+    sms = [{'kind': 'exp', 'exp_kq': 23}, {'kind': 'exp', 'exp_kq': 23, 'inv_shift': 17}]
+    if sk > 1:
+        sms.append({'kind': 'hccs', 'B': B, 'S': 1, 'Dmax': min(126, B - (256 + sk - 1) // sk), 'use_clb': sk % 2 == 0})
+    for sm in sms:
+        got = ops.attention_long(dev(q), wk, wv, 6, mode, sm, 7, mode).cpu().numpy()
+        np.testing.assert_array_equal(got, reference(oracle, q, k, v, 6, mode, sm, 7, mode))
