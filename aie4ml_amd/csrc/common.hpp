@@ -296,38 +296,35 @@ __device__ __forceinline__ int64_t floordiv64(int64_t a, int64_t b) {
     return (r != 0 && ((r < 0) != (b < 0))) ? q - 1 : q;
 }
 
-// One 16-byte chunk of an operand row for shapes the aligned kernels cannot take (K not a multiple of 16, rows that
-// are not 16-byte aligned): `rem` of its bytes belong to the row's K values, the rest read as zero, and no byte
-// past the end of the row's pitch is touched. mode 0: the chunk is aligned and lies inside the pitch; mode 1: rows
-// are 4-byte aligned with a pitch that is a multiple of 4; mode 2: neither.
-__device__ __forceinline__ v4i load_chunk_ragged(const int8_t* p, int rem, int mode) {
+// 16 bytes at any address in one instruction: vector memory accesses on this target need no alignment, and an unaligned one
+// costs what the cache lines it touches cost (8192 x 1001 -> 1000: 77 us with byte loads and branches, 25 us this way).
+typedef v4i v4i_unaligned __attribute__((aligned(1)));
+__device__ __forceinline__ v4i load16_any(const int8_t* p) { return *reinterpret_cast<const v4i_unaligned*>(p); }
+
+// Bytes s .. 15 of r moved to the front, zeros behind them (s >= 16: all zero).
+__device__ __forceinline__ v4i drop_front_bytes(v4i r, int s) {
+    const int q = s >> 2, b = s & 3;
+    if (q & 2) r = v4i{r[2], r[3], 0, 0};
+    if (q & 1) r = v4i{r[1], r[2], r[3], 0};
+    const v4i t = {static_cast<int>(__builtin_amdgcn_alignbyte(r[1], r[0], b)), static_cast<int>(__builtin_amdgcn_alignbyte(r[2], r[1], b)),
+                   static_cast<int>(__builtin_amdgcn_alignbyte(r[3], r[2], b)), static_cast<int>(__builtin_amdgcn_alignbyte(0, r[3], b))};
+    return s < 16 ? t : v4i{0, 0, 0, 0};
+}
+
+// One 16-byte chunk of an operand row of `row` bytes whose length is not a multiple of 16 or whose start is not aligned:
+// `rem` bytes of the row are left at p. A chunk that crosses the end of the row is fetched as the row's last 16 bytes
+// (no byte outside the row is touched, no branch around the load) and moved into place by chunk_in_place, which the
+// caller applies where it first uses the chunk. Rows shorter than 16 bytes are read byte by byte.
+__device__ __forceinline__ v4i load_chunk_ragged(const int8_t* p, int rem, int row) {
+    if (row >= 16) return load16_any(p + min(rem - 16, 0));
     v4i r = {0, 0, 0, 0};
-    if (rem <= 0) return r;
-    if (mode == 0) {
-        r = *reinterpret_cast<const v4i*>(p);
-    } else if (mode == 1) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (4 * j < rem) r[j] = *reinterpret_cast<const int*>(p + 4 * j);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            unsigned w = 0;
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                if (4 * j + b < rem) w |= static_cast<unsigned>(static_cast<uint8_t>(p[4 * j + b])) << (8 * b);
-            r[j] = static_cast<int>(w);
-        }
-    }
-    if (rem < 16) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int v = rem - 4 * j;  // valid bytes of this dword
-            if (v <= 0) r[j] = 0;
-            else if (v < 4) r[j] &= static_cast<int>((1u << (8 * v)) - 1u);
-        }
-    }
+    for (int b = 0; b < 15; ++b)
+        if (b < rem) r[b >> 2] |= static_cast<int>(static_cast<unsigned>(static_cast<uint8_t>(p[b])) << (8 * (b & 3)));
     return r;
+}
+__device__ __forceinline__ v4i chunk_in_place(const v4i& r, int rem, int row) {
+    return row >= 16 && rem < 16 ? drop_front_bytes(r, 16 - rem) : r;
 }
 
 // One 16-byte chunk of a row of A when A is stored transposed ([K][ld], TRANSPOSE_A of matmul.cpp:60-66 and
@@ -352,25 +349,25 @@ __device__ __forceinline__ v4i load_chunk_transposed(const int8_t* col, int64_t 
     return r;
 }
 
-// The store that goes with it: the first `rem` bytes of a 16-byte chunk, in pieces the row's alignment allows.
-__device__ __forceinline__ void store_chunk_ragged(int8_t* p, const v4i& v, int rem, int mode) {
+// The store that goes with it: the first `rem` bytes of a 16-byte chunk, at any address.
+__device__ __forceinline__ void store_chunk_ragged(int8_t* p, const v4i& v, int rem) {
+    typedef int int_unaligned __attribute__((aligned(1)));
+    typedef short short_unaligned __attribute__((aligned(1)));
     if (rem <= 0) return;
-    if (mode == 0 && rem >= 16) {
-        *reinterpret_cast<v4i*>(p) = v;
+    if (rem >= 16) {
+        *reinterpret_cast<v4i_unaligned*>(p) = v;
         return;
     }
+    int at = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int n = rem - 4 * j;  // bytes of this dword to write
-        if (n <= 0) break;
-        if (mode <= 1 && n >= 4) {
-            *reinterpret_cast<int*>(p + 4 * j) = v[j];
-        } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                if (b < n) p[4 * j + b] = static_cast<int8_t>(static_cast<unsigned>(v[j]) >> (8 * b));
+    for (int j = 0; j < 3; ++j)
+        if (4 * j + 4 <= rem) {
+            *reinterpret_cast<int_unaligned*>(p + 4 * j) = v[j];
+            at = 4 * j + 4;
         }
-    }
+    const unsigned w = static_cast<unsigned>(at == 0 ? v[0] : at == 4 ? v[1] : at == 8 ? v[2] : v[3]);
+    if (rem - at >= 2) *reinterpret_cast<short_unaligned*>(p + at) = static_cast<short>(w);
+    if ((rem - at) & 1) p[rem - 1] = static_cast<int8_t>(w >> (8 * ((rem - at) & 2)));
 }
 
 }  // namespace a4g

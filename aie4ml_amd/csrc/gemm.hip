@@ -123,7 +123,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
                 unsigned w = 0;
                 if (k < g.K && m < g.M) {
                     const int8_t* src = Ab + static_cast<int64_t>(k) * g.lda + m;
-                    if (g.ragged_a == 0 && m + 4 <= g.M) {
+                    if (g.a_dwords && m + 4 <= g.M) {
                         w = *reinterpret_cast<const unsigned*>(src);
                     } else {
 #pragma unroll
@@ -157,12 +157,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
             static_assert(!TRANS_A || RAGGED, "the transposed-A form takes B through the ragged loads");
             load_a_transposed(k0);
 #pragma unroll
-            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.ragged_b);
+            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.K);
         } else if constexpr (RAGGED) {
 #pragma unroll
-            for (int i = 0; i < Cfg::A_PER_T; ++i) ra[i] = load_chunk_ragged(pa[i] + k0, g.K - (k0 + ka[i]), g.ragged_a);
+            for (int i = 0; i < Cfg::A_PER_T; ++i) ra[i] = load_chunk_ragged(pa[i] + k0, g.K - (k0 + ka[i]), g.K);
 #pragma unroll
-            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.ragged_b);
+            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.K);
         } else {
 #pragma unroll
             for (int i = 0; i < Cfg::A_PER_T; ++i)
@@ -172,8 +172,16 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
                 rb[i] = (k0 + kb[i] < g.K) ? *reinterpret_cast<const v4i*>(pb[i] + k0) : v4i{0, 0, 0, 0};
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int buf, int k0) {
         if constexpr (TRANS_A) store_a_transposed(buf);
+        if constexpr (RAGGED) {
+            if (k0 + BK > g.K) {  // the tile that crosses K: workgroup-uniform, and no load inside
+#pragma unroll
+                for (int i = 0; i < (TRANS_A ? 0 : Cfg::A_PER_T); ++i) ra[i] = chunk_in_place(ra[i], g.K - (k0 + ka[i]), g.K);
+#pragma unroll
+                for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = chunk_in_place(rb[i], g.K - (k0 + kb[i]), g.K);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < (TRANS_A ? 0 : Cfg::A_PER_T); ++i) *reinterpret_cast<v4i*>(smem + buf * BUF + offa[i]) = ra[i];
 #pragma unroll
@@ -198,7 +206,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
 
     const int ktiles = (g.K + BK - 1) / BK;
     load_tile(0);
-    store_tile(0);
+    store_tile(0, 0);
     __syncthreads();
 
     for (int kt = 0; kt < ktiles; ++kt) {
@@ -222,7 +230,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
                     // operands swapped: the block's first index (registers) runs over n, lanes over m
                     acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], acc[i][j], 0, 0, 0);
         }
-        if (kt + 1 < ktiles) store_tile(buf ^ 1);
+        if (kt + 1 < ktiles) store_tile(buf ^ 1, (kt + 1) * BK);
         __syncthreads();
     }
 
@@ -895,36 +903,20 @@ static int env_variant() {
 #endif
 }
 
-// Shapes outside the aligned kernels' requirements: same tiles, chunk loads that respect the row ends.
-static hipError_t launch_ragged(GemmArgs g, int batch, hipStream_t stream) {
-    g.ragged_a = ragged_mode(g.A, g.lda, g.stride_a, g.K);
-    g.ragged_b = ragged_mode(g.Bt, g.ldb, g.stride_b, g.K);
-    // from two K tiles on, the pipelined kernel is ahead (25 us against 31 us at 8192 x 1024 x 1008): with descriptor loads
-    // and no branches where the activations' rows are 4-byte aligned and the other operand's 16-byte aligned rows hold
-    // K rounded up to 16 (packed weights always do) ...
-    if (g.K >= 256 && g.ragged_a <= 1 && g.ragged_b == 0 && !g.trans_a_es && static_cast<int64_t>(g.lda) >= (g.K + 3) / 4 * 4) {
-        // (8-byte aligned rows, a pitch of 1000 bytes: two loads per chunk instead of four)
-        const bool by8 = g.lda % 8 == 0 && g.stride_a % 8 == 0 && (reinterpret_cast<uintptr_t>(g.A) & 7) == 0 &&
-                         static_cast<int64_t>(g.lda) >= (g.K + 7) / 8 * 8;
-        if (by8)
-            return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, 3>(g, batch, stream)
-                                : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, 3>(g, batch, stream);
+// K off the 16-byte grid or rows at any address: same tiles, chunk loads at any address.
+static hipError_t launch_ragged(const GemmArgs& g, int batch, hipStream_t stream) {
+    // from two K tiles on the pipelined kernel is ahead (25 us against 31 us at 8192 x 1024 x 1008)
+    if (g.K < 256) return launch_tiled<128, 128, 64, 2, 2, true>(g, batch, stream);
+    if (whole_chunk_rows(g.Bt, g.ldb, g.stride_b, g.K))
         return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, 2>(g, batch, stream)
                             : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, 2>(g, batch, stream);
-    }
-    // ... else with chunk loads that respect the row ends
-    if (g.K >= 256)
-        return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, true>(g, batch, stream)
-                            : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, true>(g, batch, stream);
-    return launch_tiled<128, 128, 64, 2, 2, true>(g, batch, stream);
+    return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, 3>(g, batch, stream)
+                        : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, 3>(g, batch, stream);
 }
 
 // Left operand stored transposed ([K][lda]): the tiled kernel with the in-register tile transpose.
 static hipError_t launch_trans_a(GemmArgs g, int batch, hipStream_t stream) {
-    // ragged_a here: 0 = rows of A^T are 4-byte aligned (dword loads along m), else byte loads
-    const uintptr_t a = reinterpret_cast<uintptr_t>(g.A);
-    g.ragged_a = (g.lda % 4 == 0 && g.stride_a % 4 == 0 && a % 4 == 0) ? 0 : 2;
-    g.ragged_b = ragged_mode(g.Bt, g.ldb, g.stride_b, g.K);
+    g.a_dwords = g.lda % 4 == 0 && g.stride_a % 4 == 0 && reinterpret_cast<uintptr_t>(g.A) % 4 == 0;
     return launch_tiled<128, 128, 64, 2, 2, true, true>(g, batch, stream);
 }
 

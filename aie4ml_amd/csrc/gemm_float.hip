@@ -267,20 +267,18 @@ static hipError_t launch_float_nt(const void* A, int trans_a, int64_t lda, int64
         return launch_rs_policy<FloatPolicy<A4G_BF16>, 128, 128, 2, 2, false, false, true>(g, batch, stream);
     }
     if (!tiled) {
-        // K that does not fill its last 128-byte tile, unaligned rows: the same kernel with loads that respect the row ends
-        g.ragged_a = ragged_mode(g.A, g.lda, g.stride_a, g.K);
-        g.ragged_b = ragged_mode(g.Bt, g.ldb, g.stride_b, g.K);
-        g.trans_a_es = trans_a ? es : 0;  // A stored transposed: its chunks are gathered element by element
-        if (!trans_a && g.K >= 256 && g.ragged_a <= 1 && g.ragged_b == 0 && g.lda >= (g.K + 3) / 4 * 4) {
-            // 4-byte aligned activation rows, 16-byte aligned rows of the other operand that hold K rounded up to 16: the
-            // descriptor loads without branches (K off the 16-byte grid; the bytes past K are cleared at the staging)
-            if (fmt == A4G_F32) return launch_rs_policy<FloatPolicy<A4G_F32>, 128, 128, 2, 2, false, false, 2>(g, batch, stream);
-            if (fmt == A4G_FP8) return launch_rs_policy<FloatPolicy<A4G_FP8>, 128, 128, 2, 2, false, false, 2>(g, batch, stream);
-            return launch_rs_policy<FloatPolicy<A4G_BF16>, 128, 128, 2, 2, false, false, 2>(g, batch, stream);
-        }
-        if (fmt == A4G_F32) return launch_rs_policy<FloatPolicy<A4G_F32>, 128, 128, 2, 2, false, true>(g, batch, stream);
-        if (fmt == A4G_FP8) return launch_rs_policy<FloatPolicy<A4G_FP8>, 128, 128, 2, 2, false, true>(g, batch, stream);
-        return launch_rs_policy<FloatPolicy<A4G_BF16>, 128, 128, 2, 2, false, true>(g, batch, stream);
+        // K that does not fill its last 128-byte tile, rows at any address: the same kernel with loads at any address, or
+        // with A gathered element by element where it is stored transposed (rows shorter than 16 bytes go that way, too)
+        g.trans_a_es = trans_a ? es : 0;
+        const bool any = !trans_a && g.K >= 16, b_whole = whole_chunk_rows(g.Bt, g.ldb, g.stride_b, g.K);
+#define A4G_RAGGED_FLOAT(F)                                                                                           \
+        if (any && b_whole) return launch_rs_policy<FloatPolicy<F>, 128, 128, 2, 2, false, false, 2>(g, batch, stream); \
+        if (any) return launch_rs_policy<FloatPolicy<F>, 128, 128, 2, 2, false, false, 3>(g, batch, stream);            \
+        return launch_rs_policy<FloatPolicy<F>, 128, 128, 2, 2, false, true>(g, batch, stream);
+        if (fmt == A4G_F32) { A4G_RAGGED_FLOAT(A4G_F32) }
+        if (fmt == A4G_FP8) { A4G_RAGGED_FLOAT(A4G_FP8) }
+        A4G_RAGGED_FLOAT(A4G_BF16)
+#undef A4G_RAGGED_FLOAT
     }
     if (fmt == A4G_F32) return launch_rs_policy<FloatPolicy<A4G_F32>, 128, 128, 2, 2>(g, batch, stream);
     const int64_t tiles256 = static_cast<int64_t>((M + 255) / 256) * ((N + 255) / 256) * batch;

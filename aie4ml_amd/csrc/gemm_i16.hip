@@ -42,7 +42,6 @@ struct Gemm16Args {
     // batched use (dynamic MatMul): element strides between consecutive problems, blockIdx.y = problem
     int64_t stride_a, stride_w, stride_colsum, stride_y;
     int shift;  // used when `shifts` is null (MatMul: one host-side shift)
-    int ragged_a;  // RAGGED kernels: how chunks of A's rows may be fetched (load_chunk_ragged)
     int trans_a;   // RAGGED kernels: A is stored transposed, [K][lda]
 };
 
@@ -105,7 +104,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
             if constexpr (RAGGED)
                 ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
                                   : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                      (g.K - (k0 + kc)) * 2, g.ragged_a);
+                                                      (g.K - (k0 + kc)) * 2, g.K * 2);
             else
                 ra[i] = (k0 + kc < g.K) ? *reinterpret_cast<const v4i*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc)
                                         : v4i{0, 0, 0, 0};
@@ -118,11 +117,12 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
                                     : v4i{0, 0, 0, 0};
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int buf, int k0) {
         int8_t* st = smem + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
+            if (RAGGED && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             // eight int16 in four dwords -> their eight high bytes and eight low bytes
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             v2i hi = {static_cast<int>(__builtin_amdgcn_perm(w1, w0, 0x07050301u)), static_cast<int>(__builtin_amdgcn_perm(w3, w2, 0x07050301u))};
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
     const int ktiles = (g.K + BK - 1) / BK;
     load_tile(0);
     const int round_path = park_col_params<BN>(eg, cp, tid, col_add, col_shift);  // contains barriers
-    store_tile(0);
+    store_tile(0, 0);
     __syncthreads();
     for (int kt = 0; kt < ktiles; ++kt) {
         const int8_t* st = smem + (kt & 1) * STAGE;
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
                     acc_lo[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], al[i], acc_lo[i][j], 0, 0, 0);
                 }
         }
-        if (kt + 1 < ktiles) store_tile((kt + 1) & 1);
+        if (kt + 1 < ktiles) store_tile((kt + 1) & 1, (kt + 1) * BK);
         __syncthreads();
     }
 
@@ -233,7 +233,6 @@ struct Gemm16x16Args {
     int64_t stride_a, stride_w, stride_colsum, stride_y;  // batched use, as above
     int shift;                                            // used when `shifts` is null
     int trans_a;                                          // RAGGED kernels: A is stored transposed, [K][lda]
-    int ragged_a;                                         // RAGGED kernels: how chunks of A's rows may be fetched
 };
 
 __device__ __forceinline__ long long round_shift64(long long v, int s, int mode) {
@@ -501,7 +500,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
             if constexpr (RAGGED)
                 ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
                                   : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                      (g.K - (k0 + kc)) * 2, g.ragged_a);
+                                                      (g.K - (k0 + kc)) * 2, g.K * 2);
             else
                 ra[i] = (k0 + kc < g.K) ? *reinterpret_cast<const v4i*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc)
                                         : v4i{0, 0, 0, 0};
@@ -521,6 +520,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
+            if (RAGGED && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             // beyond K both planes are zero, so the row sums stay exact: the low bytes are biased where k < K only
             const int live = min(max(g.K - (k0 + kc), 0), 8);  // elements of this chunk below K (0 or 8 unless RAGGED)
@@ -787,7 +787,6 @@ extern "C" int a4g_dense_i16(const int16_t* A, int trans_a, int64_t lda, const i
         if (!trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A)) {
             gemm_i16i8_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
         } else {
-            g.ragged_a = ragged_mode(A, lda * 2, 0, K * 2);
             gemm_i16i8_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
         }
     } else {
@@ -853,7 +852,6 @@ extern "C" int a4g_dense_i16x16(const int16_t* A, int trans_a, int64_t lda, cons
         if (!trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A)) {
             gemm_i16i16_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
         } else {
-            g.ragged_a = ragged_mode(A, lda * 2, 0, K * 2);
             gemm_i16i16_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
         }
     } else {
@@ -925,7 +923,6 @@ extern "C" int a4g_matmul_i16(const int16_t* A, int trans_a, int64_t lda, int64_
         if (tiled) {
             gemm_i16i16_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
         } else {  // the packed planes in the workspace are always aligned and zero padded; A is fetched as its rows allow
-            g.ragged_a = ragged_mode(A, lda * 2, stride_a * 2, K * 2);
             gemm_i16i16_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
         }
     } else {
@@ -948,7 +945,6 @@ extern "C" int a4g_matmul_i16(const int16_t* A, int trans_a, int64_t lda, int64_
         if (tiled) {
             gemm_i16i8_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
         } else {
-            g.ragged_a = ragged_mode(A, lda * 2, stride_a * 2, K * 2);
             gemm_i16i8_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
         }
     }

@@ -61,9 +61,7 @@ struct GemmArgs {
     int out_kind;
     int mode;
     const int8_t* Bt_lo;    // second byte plane of B^T (policies with SPLIT_B), same pitch and strides as Bt
-    // only read by the ragged form of the tiled int8 kernel: how a 16-byte chunk of an operand row may be fetched
-    // (0 = one aligned load inside the row pitch, 1 = dwords, 2 = bytes); bytes at or past K always read as zero
-    int ragged_a, ragged_b;
+    int a_dwords;  // only read by the transposed-A form of the tiled int8 kernel: rows of A^T are 4-byte aligned
     // only read by the ragged forms of gemm_rs_kernel: 0, or the element size in bytes of an A that is stored transposed
     // ([K][lda]: lda, stride_a and K stay in bytes, K in bytes of a row of the untransposed operand)
     int trans_a_es;
@@ -110,13 +108,12 @@ __device__ __forceinline__ TileCoord tile_coord(const GemmArgs& g) {
 }
 
 // Copies the LDS image of an output tile (row pitch BN * obytes + 16) to global memory, whole rows in
-// 16-byte pieces; pieces that cross the matrix edge or a misaligned pitch go byte by byte.
+// 16-byte pieces at any address; the piece that crosses the matrix edge goes in 4-, 2- and 1-byte stores.
 template <int BM, int BN, int NT>
 __device__ __forceinline__ void store_tile_image(const GemmArgs& g, const TileCoord& tc, const int8_t* smem, int obytes, int tid) {
     const int cpitch = BN * obytes + 16;
     int8_t* Cb = static_cast<int8_t*>(g.C) + tc.batch * g.stride_c * obytes;
     const int cpr = BN * obytes / 16;  // 16-byte chunks per tile row
-    const bool vec_ok = ((g.ldc * obytes) % 16 == 0) && ((reinterpret_cast<uintptr_t>(Cb) & 15) == 0);
     for (int idx = tid; idx < BM * cpr; idx += NT) {
         const int row = idx / cpr, ch = idx % cpr;
         const int m = tc.m0 + row;
@@ -124,13 +121,7 @@ __device__ __forceinline__ void store_tile_image(const GemmArgs& g, const TileCo
         if (m >= g.M || nb >= g.N * obytes) continue;
         const v4i v = *reinterpret_cast<const v4i*>(smem + row * cpitch + ch * 16);
         int8_t* dst = Cb + static_cast<int64_t>(m) * g.ldc * obytes + nb;
-        if (vec_ok && nb + 16 <= g.N * obytes) {
-            *reinterpret_cast<v4i*>(dst) = v;
-        } else {
-            const int nbytes = min(16, g.N * obytes - nb);
-            const int8_t* srcb = smem + row * cpitch + ch * 16;
-            for (int b = 0; b < nbytes; ++b) dst[b] = srcb[b];
-        }
+        store_chunk_ragged(dst, v, g.N * obytes - nb);
     }
 }
 
@@ -187,22 +178,21 @@ struct RsCfg {
                   "plane split: a wave's rows must hold whole high/low runs");
 };
 
-// How the ragged kernels may fetch 16-byte chunks of an operand's rows (see load_chunk_ragged).
-static inline int ragged_mode(const void* p, int64_t ld, int64_t stride, int64_t K) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-    if (ld % 16 == 0 && stride % 16 == 0 && a % 16 == 0 && ld >= (K + 15) / 16 * 16) return 0;
-    if (ld % 4 == 0 && stride % 4 == 0 && a % 4 == 0) return 1;
-    return 2;
+// Whether an operand's rows are 16-byte aligned and their pitch holds K rounded up to 16 bytes (packed weights always).
+static inline bool whole_chunk_rows(const void* p, int64_t ld, int64_t stride, int64_t K) {
+    return ld % 16 == 0 && stride % 16 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld >= (K + 15) / 16 * 16;
 }
 
-// RAGGED: K need not fill its last tile and rows need not be aligned (chunk loads that respect the row ends).
+// RAGGED: A stored transposed, or rows shorter than 16 bytes.
 // KTAIL: aligned rows, K in whole 16-byte chunks but not whole tiles: the aligned form's descriptor loads, with the
 // chunks past K sent to an offset outside the descriptor (they read as zero) - no load sits in a branch, so the waits
 // stay exact, which the ragged loads' branches do not allow (8192 x 784 -> 128: 17 us ragged, 9 us this way).
-// KTAIL 2: the same for K off the 16-byte grid: rows of A 4-byte aligned (four dword loads per chunk, each inside K or
-// sent outside the descriptor), rows of B 16-byte aligned with a pitch that holds K rounded up to 16; the bytes past K
-// of the one dword or chunk that straddles it are cleared where the last K tile is staged. KTAIL 3: the same with rows
-// of A 8-byte aligned, two 8-byte loads per chunk.
+// KTAIL 2: any K of at least 16 bytes and rows of A at any address: one 16-byte load per chunk wherever it lies
+// (vector loads need no alignment); the chunk that crosses the end of a row is fetched as the row's last 16 bytes and moved
+// into place where the last K tile is staged (a workgroup-uniform branch around vector arithmetic only). Rows of B are
+// 16-byte aligned with a pitch that holds K rounded up to 16; KTAIL 3: rows of B at any address as well.
+// 8192 x 1001 -> 1000 int8: 77 us with byte loads in branches, 25 us this way (bfloat16 147 and 38, fp8 81 and 28); 8192 x 1000
+// -> 1000: 24.5 us with two 8-byte loads per chunk, 22.3 us.
 template <class P, int BM, int BN, int WAVES_M, int WAVES_N, bool EARLY = false, bool RAGGED = false, int KTAIL = 0>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_rs_kernel(GemmArgs g) {
     static_assert(KTAIL == 0 || (!RAGGED && !P::SPLIT_A && !P::SPLIT_B), "the K tail form serves the unsplit policies");
@@ -254,11 +244,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_rs_kernel(GemmArgs
     // policies, short of registers, reloaded address pairs from scratch inside the loop, each reload waiting for every
     // load in flight.
     constexpr int A_TILE_BYTES = P::SPLIT_A ? 2 * BK : BK;
-    // KTAIL 2 reads the dword (A) or chunk (B) that straddles K whole: inside the row's pitch, which the host has checked
-    const int64_t a_range = static_cast<int64_t>(g.M - 1 - m0) * g.lda +
-                            (KTAIL == 3 ? (g.K + 7) / 8 * 8 : KTAIL == 2 ? (g.K + 3) / 4 * 4 : KTAIL ? g.K : static_cast<int64_t>(g.K / BK) * A_TILE_BYTES);
+    const int64_t a_range = static_cast<int64_t>(g.M - 1 - m0) * g.lda + (KTAIL ? g.K : static_cast<int64_t>(g.K / BK) * A_TILE_BYTES);
     const int64_t b_range = static_cast<int64_t>(g.N - 1 - n0) * g.ldb +
-                            (KTAIL >= 2 ? (g.K + 15) / 16 * 16 : KTAIL ? g.K : static_cast<int64_t>(g.K / BK) * BK);
+                            (KTAIL == 2 ? (g.K + 15) / 16 * 16 : KTAIL ? g.K : static_cast<int64_t>(g.K / BK) * BK);
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(Abase), 0, static_cast<int>(a_range < 0x7fffffff ? a_range : 0x7fffffff), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b =
@@ -268,32 +256,17 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_rs_kernel(GemmArgs
     const int voff_b = lrow * static_cast<int>(g.ldb) + lchunk * 16;
     auto load_one = [&](int kt, int idx) {
         if constexpr (KTAIL != 0) {
-            constexpr unsigned NOWHERE = 0xfffffff0u;  // beyond every descriptor: reads as zero
-            const bool inside = kt * BK + lchunk * 16 < g.K;
+            constexpr unsigned NOWHERE = 0x80000000u;  // beyond every descriptor, whatever is added: reads as zero
+            const int k = kt * BK + lchunk * 16;
+            const bool inside = k < g.K;
             if (idx < Cfg::A_LOADS) {
-                const unsigned off = voff_a + kt * BK + idx * Cfg::ROWS_PER_PASS * static_cast<int>(g.lda);
-                if constexpr (KTAIL == 3) {
-                    typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
-                    const int rem = g.K - (kt * BK + lchunk * 16);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const v2u_t w = __builtin_amdgcn_raw_buffer_load_b64(rsrc_a, 8 * j < rem ? off + 8 * j : NOWHERE, 0, 0);
-                        ra[idx][2 * j] = static_cast<int>(w[0]);
-                        ra[idx][2 * j + 1] = static_cast<int>(w[1]);
-                    }
-                    return;
-                }
-                if constexpr (KTAIL == 2) {
-                    const int rem = g.K - (kt * BK + lchunk * 16);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        ra[idx][j] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rsrc_a, 4 * j < rem ? off + 4 * j : NOWHERE, 0, 0));
-                    return;
-                }
-                ra[idx] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, inside ? off : NOWHERE, 0, 0));
+                const int at = KTAIL >= 2 ? min(k, g.K - 16) : k;
+                const unsigned off = (inside ? static_cast<unsigned>(lrow * static_cast<int>(g.lda) + at) : NOWHERE) + idx * Cfg::ROWS_PER_PASS * static_cast<int>(g.lda);
+                ra[idx] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, 0, 0));
             } else {
-                const unsigned off = voff_b + kt * BK + (idx - Cfg::A_LOADS) * Cfg::ROWS_PER_PASS * static_cast<int>(g.ldb);
-                rb[idx - Cfg::A_LOADS] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, inside ? off : NOWHERE, 0, 0));
+                const int at = KTAIL == 3 ? min(k, g.K - 16) : k;
+                const unsigned off = (inside ? static_cast<unsigned>(lrow * static_cast<int>(g.ldb) + at) : NOWHERE) + (idx - Cfg::A_LOADS) * Cfg::ROWS_PER_PASS * static_cast<int>(g.ldb);
+                rb[idx - Cfg::A_LOADS] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, off, 0, 0));
             }
             return;
         }
@@ -307,8 +280,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_rs_kernel(GemmArgs
                 ra[idx] = load_chunk_transposed(g.A + tc.batch * g.stride_a + static_cast<int64_t>(m) * es, g.lda, (kt * BK + lchunk * 16) / es, g.K / es, es);
                 return;
             }
-            if (idx < Cfg::A_LOADS) ra[idx] = load_chunk_ragged(Abase + offa[idx] + static_cast<int64_t>(kt) * BK, rem, g.ragged_a);
-            else rb[idx - Cfg::A_LOADS] = load_chunk_ragged(Bbase + offb[idx - Cfg::A_LOADS] + static_cast<int64_t>(kt) * BK, rem, g.ragged_b);
+            if (idx < Cfg::A_LOADS) ra[idx] = load_chunk_ragged(Abase + offa[idx] + static_cast<int64_t>(kt) * BK, rem, g.K);
+            else rb[idx - Cfg::A_LOADS] = load_chunk_ragged(Bbase + offb[idx - Cfg::A_LOADS] + static_cast<int64_t>(kt) * BK, rem, g.K);
             return;
         }
         if constexpr (P::SPLIT_B) {
@@ -326,17 +299,23 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_rs_kernel(GemmArgs
         }
     };
     const int ktiles = (RAGGED || KTAIL != 0) ? (g.K + BK - 1) / BK : g.K / BK;
-    int stage_kt = 0;  // the K tile that the staging registers hold (KTAIL 2: its last tile is cleared past K)
+    int stage_kt = 0;  // the K tile that the staging registers hold (its last one is put in order past K)
     auto store_one = [&](int8_t* stage, int idx) {
-        if constexpr (KTAIL >= 2) {
+        if constexpr (KTAIL >= 2 || RAGGED) {
             if (stage_kt == ktiles - 1) {  // workgroup-uniform, and no load inside
                 const int rem = g.K - (stage_kt * BK + lchunk * 16);
-                v4i& r = idx < Cfg::A_LOADS ? ra[idx] : rb[idx - Cfg::A_LOADS];
+                if (idx < Cfg::A_LOADS) {
+                    if (!RAGGED || !g.trans_a_es) ra[idx] = chunk_in_place(ra[idx], rem, g.K);
+                } else if (KTAIL == 2) {  // what lies between K and the next chunk is not the operand's
+                    v4i& r = rb[idx - Cfg::A_LOADS];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int v = rem - 4 * j;  // bytes of this dword that belong to K
-                    if (v <= 0) r[j] = 0;
-                    else if (v < 4) r[j] &= static_cast<int>((1u << (8 * v)) - 1u);
+                    for (int j = 0; j < 4; ++j) {
+                        const int v = rem - 4 * j;  // bytes of this dword that belong to K
+                        if (v <= 0) r[j] = 0;
+                        else if (v < 4) r[j] &= static_cast<int>((1u << (8 * v)) - 1u);
+                    }
+                } else {
+                    rb[idx - Cfg::A_LOADS] = chunk_in_place(rb[idx - Cfg::A_LOADS], rem, g.K);
                 }
             }
         }

@@ -622,11 +622,11 @@ __device__ __forceinline__ int max_i8x4(unsigned w) {
 // l, l+L, ... (NCH of them), 16 int8 each.
 // FASTP: uint8 output that needs no clamp with a shift of at most 16: the probability is read as byte 2 of
 // score * (inv << (16 - shift)), which saves the shift. FULL: cols == L * NCH * 16, no chunk is ever masked.
-// RAGGED (never with FULL): cols need not be a multiple of 16 nor rows 16-byte aligned; `ragged` says how a row's
-// chunks may be fetched and stored (load_chunk_ragged), the last chunk of a row is cut at cols.
+// RAGGED (never with FULL): cols need not be a multiple of 16 nor rows 16-byte aligned (load_chunk_ragged), the last chunk
+// of a row is cut at cols.
 template <int L, int NCH, bool FASTP, bool FULL, bool RAGGED = false>
 __global__ __launch_bounds__(256) void softmax_lut_kernel(const int8_t* __restrict__ x, void* __restrict__ out, int rows,
-                                                           int cols, SoftmaxParams p, int ragged = 0) {
+                                                           int cols, SoftmaxParams p) {
     static_assert(!(RAGGED && FULL), "a ragged row never fills its chunks");
     __shared__ int table[256];
     table[threadIdx.x] = table_entry(p, threadIdx.x);
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256) void softmax_lut_kernel(const int8_t* __restri
             if constexpr (RAGGED) {
                 if (valid[i]) {
                     const int rem = cols - col0;
-                    xv[i] = load_chunk_ragged(x + base + col0, rem, ragged);
+                    xv[i] = chunk_in_place(load_chunk_ragged(x + base + col0, rem, cols), rem, cols);
 #pragma unroll
                     for (int w = 0; w < 4; ++w) {  // bytes past the row's end: -128, which no maximum notices
                         const int n = rem - 4 * w;
@@ -730,9 +730,8 @@ __global__ __launch_bounds__(256) void softmax_lut_kernel(const int8_t* __restri
                 if constexpr (RAGGED) {
                     int8_t* dst = reinterpret_cast<int8_t*>(static_cast<int16_t*>(out) + base + col0);
                     const int rem = (cols - col0) * 2;  // bytes
-                    const int mode = ragged == 0 ? 1 : ragged;  // two-byte elements: an aligned byte row gives aligned dwords at best
-                    store_chunk_ragged(dst, o[0], rem, (cols % 2 == 0 && mode == 1) ? 1 : 2);
-                    store_chunk_ragged(dst + 16, o[1], rem - 16, (cols % 2 == 0 && mode == 1) ? 1 : 2);
+                    store_chunk_ragged(dst, o[0], rem);
+                    store_chunk_ragged(dst + 16, o[1], rem - 16);
                 } else {
                     v4i* dst = reinterpret_cast<v4i*>(static_cast<int16_t*>(out) + base + col0);
                     __builtin_nontemporal_store(o[0], dst);
@@ -756,7 +755,7 @@ __global__ __launch_bounds__(256) void softmax_lut_kernel(const int8_t* __restri
                     }
                 }
                 if constexpr (RAGGED)
-                    store_chunk_ragged(static_cast<int8_t*>(out) + base + col0, o, cols - col0, ragged);
+                    store_chunk_ragged(static_cast<int8_t*>(out) + base + col0, o, cols - col0);
                 else
                     __builtin_nontemporal_store(o, reinterpret_cast<v4i*>(static_cast<uint8_t*>(out) + base + col0));
             }
@@ -801,12 +800,12 @@ __global__ __launch_bounds__(256) void softmax_generic_kernel(const int8_t* __re
 
 template <int L, int NCH>
 static void launch_softmax(bool noclamp, int grid, hipStream_t stream, const int8_t* x, void* out, int rows, int cols,
-                           const SoftmaxParams& p, int ragged) {
+                           const SoftmaxParams& p, bool ragged) {
     const bool fastp = noclamp && !p.out_i16 && p.out_shift <= 16;
-    if (ragged >= 0) {
+    if (ragged) {
         if constexpr (NCH <= 4) {  // the ragged form stops at 4096 columns
-            if (fastp) softmax_lut_kernel<L, NCH, true, false, true><<<grid, 256, 0, stream>>>(x, out, rows, cols, p, ragged);
-            else softmax_lut_kernel<L, NCH, false, false, true><<<grid, 256, 0, stream>>>(x, out, rows, cols, p, ragged);
+            if (fastp) softmax_lut_kernel<L, NCH, true, false, true><<<grid, 256, 0, stream>>>(x, out, rows, cols, p);
+            else softmax_lut_kernel<L, NCH, false, false, true><<<grid, 256, 0, stream>>>(x, out, rows, cols, p);
         }
         return;
     }
@@ -827,13 +826,7 @@ static int softmax_dispatch(const int8_t* x, void* out, int64_t rows, int64_t co
     A4G_REQUIRE(x && out, A4G_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
     const bool aligned = cols % 16 == 0 && aligned16(x) && aligned16(out);
     if (cols <= 4096 || (aligned && cols <= 16384)) {
-        // rows off the 16-byte grid: the same kernel with loads and stores that respect the row ends; the output has
-        // the input's row offsets, so one mode serves both when both bases are equally aligned
-        int ragged = -1;
-        if (!aligned) {
-            const uintptr_t both = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out);
-            ragged = (cols % 4 == 0 && both % 4 == 0) ? 1 : 2;
-        }
+        const bool ragged = !aligned;  // rows off the 16-byte grid: the same kernel with loads and stores at any address
         const int chunks = static_cast<int>((cols + 15) / 16);
         // lanes per row: smallest power of two >= chunks (capped at 64), then chunks per lane
         int L = 1;

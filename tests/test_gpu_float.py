@@ -155,3 +155,22 @@ def test_float_argument_errors(ops):
         ops.dense_float(torch.zeros((2, 8), dtype=torch.float32, device='cuda'), p)
     with pytest.raises(ValueError, match='features'):
         ops.dense_float(torch.zeros((2, 9), dtype=torch.bfloat16, device='cuda'), p)
+
+
+@pytest.mark.parametrize('fmt', ['bfloat16', 'fp8_e4m3', 'float32'])
+@pytest.mark.parametrize('K', [3, 7, 8, 9, 17, 33, 131, 300])
+def test_dense_float_rows_at_any_address(ops, oracle, fmt, K):
+    """A column window of a wider matrix whose other columns hold NaN: rows at any address, K around 16 bytes of operand and
+    a K tile. Small integers, so every order of summation gives the same bits."""
+    r = np.random.default_rng(K)
+    A, W = (r.integers(-2, 3, sh).astype(np.float32) for sh in ((70, K), (K, 37)))
+    t = {'bfloat16': torch.bfloat16, 'fp8_e4m3': torch.float8_e4m3fn, 'float32': torch.float32}[fmt]
+    wide = torch.full((70, K + 3), float('nan')).to(t)
+    wide[:, 1:K + 1] = torch.from_numpy(A).to(t)
+    p = ops.pack_dense_float(torch.from_numpy(W).to(t).cuda(), None)
+    got = ops.dense_float(wide.cuda()[:, 1:K + 1], p).float().cpu()
+    want = torch.from_numpy(A @ W)  # exact; fp8 results up to 16 are, larger ones round to even or away from zero at ties
+    if fmt == 'fp8_e4m3':
+        exact = want.abs() <= 16
+        got, want = got[exact], want[exact]
+    assert torch.equal(got, want if fmt == 'float32' else want.to(t).float())

@@ -668,6 +668,28 @@ def test_dense_ragged_reduction_and_unaligned_rows(ops, oracle, kind, case):
         assert np.array_equal(got, oracle.dense(A, W, bias, shifts, mode, relu=relu, out=out)), (mode, relu)
 
 
+@pytest.mark.parametrize('K', [1, 15, 16, 17, 63, 65, 79, 255, 256, 257, 271, 385])
+@pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
+def test_dense_chunk_that_crosses_the_end_of_a_row(ops, oracle, kind, K):
+    """Rows at every address modulo 16, K around 16 bytes, a K tile and two of them: the chunk that crosses a row's end is
+    fetched as the row's last 16 bytes and moved into place; results of 1 to 15 columns past a 16-byte piece leave in 4-,
+    2- and 1-byte stores. Window and result lie between extreme values that must neither count nor change."""
+    r = rng(K + 7 * len(kind))
+    adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
+    info = np.iinfo(adt)
+    for M, N, off in ((130, 131, K % 16), (37, 13, 5), (1, 1, 0)):
+        wide = np.where(np.arange(off + K + 3) % 2, info.max, info.min).astype(adt)[None].repeat(M, 0)
+        A = wide[:, off:off + K] = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+        W = r.integers(-32768, 32768, (K, N)).astype(np.int16) if kind == 'int16x16' else gauss8(r, 40, (K, N))
+        p = ops.pack_dense(dev(W), None, 20 if kind == 'int16x16' else 10)
+        out = 'int16' if kind.startswith('int16') else 'int8'
+        y = dev(np.full((M, N + 3), 77, np.int16 if out == 'int16' else np.int8))
+        ops.dense(dev(wide)[:, off:off + K], p, 'conv_even', out_kind=out, out=y[:, 1:N + 1])
+        got = host(y)
+        assert np.array_equal(got[:, 1:N + 1], oracle.dense(A, W, None, np.array([20 if kind == 'int16x16' else 10]), 'conv_even', out=out)), (M, N)
+        assert (got[:, 0] == 77).all() and (got[:, N + 1:] == 77).all(), (M, N)
+
+
 @pytest.mark.parametrize('case', [(300, 200, 784, 16), (1, 128, 784, 0), (1000, 130, 800, 240), (700, 520, 272, 112),
                                   (4096, 4096, 1040, 0), (4100, 4096, 528, 16)])
 @pytest.mark.parametrize('a_dtype', [np.int8, np.uint8])
