@@ -16,7 +16,7 @@ LIB_PATH = Path(__file__).resolve().parent / 'libaie4ml_gfx950.so'
 # measurement aids of bench.py (the matrix-core calibration loop), kept out of the library an integrator ships
 BENCH_LIB_PATH = Path(__file__).resolve().parent / 'libaie4ml_bench_gfx950.so'
 BENCH_SOURCES = ('calib.hip',)
-SOURCES = ('abi.hip', 'rowops.hip', 'gemm.hip', 'mlp.hip', 'attention.hip', 'attention_long.hip', 'matmul_lean.hip', 'gemm_i16.hip', 'gemm_float.hip', 'gemm_wreg.hip', 'gemm_wrow.hip', 'gemm_wrow_plain.hip', 'gemm_wrow_sym_inf.hip', 'gemm_wrow_conv_even.hip', 'gemm_sk.hip', 'gemm_rowln.hip')
+SOURCES = ('abi.hip', 'rowops.hip', 'gemm.hip', 'mlp.hip', 'attention.hip', 'attention_long.hip', 'matmul_lean.hip', 'gemm_i16.hip', 'gemm_float.hip', 'gemm_wreg.hip', 'gemm_wrow.hip', 'gemm_wrow_plain.hip', 'gemm_wrow_sym_inf.hip', 'gemm_wrow_conv_even.hip', 'gemm_sk.hip', 'gemm_few.hip', 'gemm_rowln.hip')
 
 HIPCC_FLAGS = [
     '--offload-arch=gfx950',

@@ -15,6 +15,7 @@
 #include "common.hpp"
 #include "gemm_direct.hpp"
 #include "gemm_epilogue.hpp"
+#include "gemm_few.hpp"
 #include "gemm_rs.hpp"
 #include "matmul_lean.hpp"
 
@@ -993,6 +994,8 @@ static int dense_i8(const char* who, const void* A, int a_kind, int trans_a, int
     hipError_t e;
     if (trans_a) {
         e = launch_trans_a(g, 1, stream);
+    } else if (few_preferred(g, FEW_I8, 1)) {
+        e = launch_few(g, FEW_I8, 1, stream);
     } else if (tiled && wreg_applicable(g)) {
         e = launch_wreg(g, stream);
     } else if (tiled && sk_applicable(g) && sk_preferred(g)) {

@@ -174,3 +174,17 @@ def test_dense_float_rows_at_any_address(ops, oracle, fmt, K):
         exact = want.abs() <= 16
         got, want = got[exact], want[exact]
     assert torch.equal(got, want if fmt == 'float32' else want.to(t).float())
+
+
+@pytest.mark.parametrize('fmt', FORMATS)
+@pytest.mark.parametrize('M,K,N', [(1, 32, 8), (16, 1000, 40), (17, 129, 129), (64, 2048, 1024), (130, 96, 770), (512, 1536, 1024)])
+def test_dense_float_with_few_output_tiles(ops, oracle, fmt, M, K, N):
+    """The kernel for small outputs in the floating-point formats: every tile form, K on and off its tiles, bias and ReLU,
+    against the oracle's exact sums within the bound on a float32 dot product in any order plus one rounding."""
+    r = np.random.default_rng(M + K + N)
+    A, W = operand(r, (M, K), fmt, oracle), operand(r, (K, N), fmt, oracle, 1.0 / np.sqrt(K))
+    b = r.normal(0, 1, N).astype(np.float32)
+    p = ops.pack_dense_float(dev(W, fmt), torch.from_numpy(b).cuda())
+    for relu in (False, True):
+        got = host(ops.dense_float(dev(A, fmt), p, relu=relu))
+        check(got, oracle.dense_float(A, W, b, relu=relu, fmt=fmt), fmt, K, np.abs(A).astype(np.float64) @ np.abs(W) + np.abs(b))

@@ -668,6 +668,28 @@ def test_dense_ragged_reduction_and_unaligned_rows(ops, oracle, kind, case):
         assert np.array_equal(got, oracle.dense(A, W, bias, shifts, mode, relu=relu, out=out)), (mode, relu)
 
 
+@pytest.mark.parametrize('M,N,K', [(1, 1, 16), (1, 17, 1024), (15, 33, 40), (16, 16, 128), (17, 48, 640), (33, 160, 129), (40, 1030, 513),
+                                   (64, 4096, 2048), (130, 770, 1000), (300, 47, 137), (1000, 64, 1152), (512, 2048, 3072)])
+@pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
+def test_dense_with_few_output_tiles(ops, oracle, kind, M, N, K):
+    """The kernel for small outputs: every tile form (16 x 16 to 64 x 64), rows and columns off their edges, reductions
+    below one K tile, off and on its grid, shorter and longer than the waves' shares, every output type, per-channel
+    shifts that include 0 and the largest, and accumulators that wrap."""
+    r = rng(M + N + K + len(kind))
+    adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
+    info = np.iinfo(adt)
+    A = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+    W = r.integers(-32768, 32768, (K, N)).astype(np.int16) if kind == 'int16x16' else gauss8(r, 40, (K, N))
+    bias = r.integers(-2**31, 2**31, N).astype(np.int32)
+    top = 30 if kind == 'int16x16' else (20 if kind == 'int16x8' else 12)
+    shifts = r.integers(top - 5, top + 1, N).astype(np.int32)
+    shifts[:3] = [0, 62 if kind == 'int16x16' else 31, 1][:N]
+    p = ops.pack_dense(dev(W), dev(bias), shifts)
+    for mode, relu, out in (('conv_even', True, 'int8'), ('symmetric_inf', False, 'int16'), ('floor', True, 'uint8'), ('conv_odd', False, 'int8')):
+        got = host(ops.dense(dev(A), p, mode, relu=relu, out_kind=out))
+        assert np.array_equal(got, oracle.dense(A, W, bias, shifts, mode, relu=relu, out=out)), (mode, relu, out)
+
+
 @pytest.mark.parametrize('K', [1, 15, 16, 17, 63, 65, 79, 255, 256, 257, 271, 385])
 @pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
 def test_dense_chunk_that_crosses_the_end_of_a_row(ops, oracle, kind, K):
