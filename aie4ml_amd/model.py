@@ -132,8 +132,6 @@ class GPUModel:
             raise ValueError(f'Unknown simulator "{simulator}". Expected one of: gpu.')
         if not self._compiled:
             self.compile()
-        import torch
-
         prepared = self.prepare_inputs(X, quantize=quantize_in)
         graph = self.context.ir.logical
         dev_inputs = self.to_device(prepared)
@@ -147,8 +145,7 @@ class GPUModel:
             dev_out = captured(dev_inputs)
         else:
             dev_out = self.execute(dev_inputs, batch_scale=iters)
-        torch.cuda.synchronize()
-        results = {}
+        results = {}  # each copy to the host below waits for the stream that the launches went to
         for t in graph.graph_outputs():
             dtype = self._io_dtype(t, 'output')
             if dtype.is_float:
@@ -174,7 +171,7 @@ class GPUModel:
         plan = {'add_layernorm': plan.get('add_layernorm', {}), 'mlp_chains': plan.get('mlp_chains', []),
                 'attention': plan.get('attention', []), 'dense_add_layernorm': plan.get('dense_add_layernorm', {}),
                 'mlp_add_layernorm': plan.get('mlp_add_layernorm', {})}
-        values: Dict[str, Any] = dict(inputs)
+        values = _Values(inputs)
         fused_ln = {v['layer_norm'] for v in plan['add_layernorm'].values()}
         fused_ln |= {v['layer_norm'] for v in plan['dense_add_layernorm'].values()}
         fused_ln |= {v['layer_norm'] for v in plan['mlp_add_layernorm'].values()}
@@ -182,8 +179,8 @@ class GPUModel:
         fused_dense |= {n for v in plan['mlp_add_layernorm'].values() for n in v['chain']}  # run at the add's position
         chain_head = {c[0]: c for c in plan['mlp_chains']}
         chain_rest = {n for c in plan['mlp_chains'] for n in c[1:]}
-        attn_at, attn_skip = {}, set()
-        order = {n.name: i for i, n in enumerate(graph.nodes)}
+        attn_at, attn_skip, merged = {}, set(), set()
+        order = {n.name: i for i, n in enumerate(graph.nodes)} if plan['attention'] else {}
         for grp in plan['attention']:
             members = [tr[k] for tr in grp['heads'] for k in ('qk', 'softmax', 'pv')]
             first = min((tr['qk'] for tr in grp['heads']), key=order.get)
@@ -191,6 +188,7 @@ class GPUModel:
             attn_skip.update(m for m in members if m != first)
             if grp.get('concat'):
                 attn_skip.add(grp['concat'])
+                merged.update(tr[k] for tr in grp['heads'] for k in ('q', 'k', 'v'))
 
         def launch(label, kind, members, fn):
             if trace is None:
@@ -208,7 +206,7 @@ class GPUModel:
             if node.name in attn_skip:
                 continue
             if node.is_placeholder:
-                self._run_view(node, values)
+                self._run_view(node, values, merged)
                 continue
             if node.name in fused_ln or node.name in fused_dense or node.name in chain_rest:
                 continue  # executed as part of a fused launch
@@ -242,14 +240,22 @@ class GPUModel:
                 launch(node.name, node.op_type, [node.name], lambda: values.update(inst.variant.run(inst, args)))
         return {name: values[name] for name in graph.output_tensor_names}
 
-    def _run_view(self, node, values) -> None:
+    def _run_view(self, node, values, merged=()) -> None:
+        """`merged`: the operands of attention groups that run as one launch over all heads. Those read the heads from their
+        common source, so a slice that has no other reader is made when something asks for it (36 views of an encoder
+        block with 12 heads: 50 of the 205 us its call spent on the host)."""
         from . import ops
 
         sv, cv = node.traits.get('slice_view'), node.traits.get('concat_view')
         if sv is not None:
-            src = values[sv.data['source']]
+            src, axis = values[sv.data['source']], int(sv.data['axis'])
+            tensors = self.context.ir.logical.tensors
             for item in sv.data['slices']:
-                values[item['output']] = src.narrow(int(sv.data['axis']), int(item['start']), int(item['extent']))
+                name = item['output']
+                if name in merged and len(tensors[name].consumers) == 1:
+                    values.windows[name] = (src, axis, item)
+                else:
+                    values[name] = src.narrow(axis, int(item['start']), int(item['extent']))
         elif cv is not None:
             values[cv.data['output']] = ops.concat([values[i['input']] for i in cv.data['slices']], int(cv.data['axis']))
         elif node.op_type == 'input':
@@ -336,8 +342,11 @@ class GPUModel:
             nh, d = len(grp['heads']), int(self.context.ir.logical.tensors[tr0['q']].shape[-1])
 
             def heads_view(t, base):  # [batch, seq, H*d] slice -> [batch, H, seq, d] view
-                t = t.narrow(-1, base, nh * d)
-                return t.unflatten(-1, (nh, d)).permute(0, 2, 1, 3)
+                if base or t.shape[-1] != nh * d:
+                    t = t.narrow(-1, base, nh * d)
+                batch, seq, _ = t.shape
+                sb, ss, s1 = t.stride()
+                return t.as_strided((batch, nh, seq, d), (sb, d * s1, ss, s1))
 
             q = heads_view(values[grp['q_src']], grp['q_base'])
             k = heads_view(values[grp['k_src']], grp['k_base'])
@@ -349,7 +358,7 @@ class GPUModel:
             out = torch.empty((q.shape[0], q.shape[2], nh * d), dtype=torch.int8, device=q.device)
             attend = ops.attention_long if ops.attention_is_long(d, int(k.shape[-2])) else ops.attention
             attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode,
-                   out=out.unflatten(-1, (nh, d)).permute(0, 2, 1, 3))
+                   out=heads_view(out, 0))
             values[grp['out']] = out
         elif not _views_are_16_byte_aligned(values[tr0['q']], values[tr0['k']], values[tr0['v']]):
             self._run_attention_unfused(grp, values)
@@ -394,10 +403,29 @@ class GPUModel:
         values[insts[-1].node.outputs[0].name] = y.reshape(lead + (y.shape[-1],))
 
 
+class _Values(dict):
+    """Tensor name -> device tensor of one pass, and the slices that are made on first use."""
+
+    def __init__(self, inputs: Dict[str, Any]):
+        super().__init__(inputs)
+        self.windows: Dict[str, Any] = {}  # tensor name -> (source, axis, the slice of it)
+
+    def __missing__(self, name: str):
+        src, axis, item = self.windows[name]  # KeyError for a tensor that nothing has produced, as in a plain dict
+        self[name] = view = src.narrow(axis, int(item['start']), int(item['extent']))
+        return view
+
+
 def _views_are_16_byte_aligned(*tensors) -> bool:
     """What the fused attention launch asks of its operands: 16-byte aligned base addresses and row / head / batch
     pitches (int8 tensors, so elements are bytes)."""
-    return all(t.data_ptr() % 16 == 0 and all(int(st) % 16 == 0 for st in t.stride()[:-1]) for t in tensors)
+    for t in tensors:
+        at = t.data_ptr()
+        for st in t.stride()[:-1]:
+            at |= st  # (a power of two divides all of them if it divides their bitwise or)
+        if at % 16:
+            return False
+    return True
 
 
 def _mlp_layers_are_faster(rows: int, layers, on_matrix_units: bool = False) -> bool:

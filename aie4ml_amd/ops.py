@@ -40,7 +40,7 @@ def _dev(t: torch.Tensor, name: str) -> torch.Tensor:
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None  # (the entry points declare c_void_p and take the number as it is)
 
 
 def _pitched_rows(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -58,8 +58,24 @@ def _pitch(t2: torch.Tensor) -> int:
     return int(t2.stride(0)) if t2.shape[0] > 1 else int(t2.shape[1])
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    """The current device's current stream as the number the entry points take. torch.cuda.current_stream() builds a
+    Stream object around it on every call (4 us of the 13 us that a small Dense call spent on the host)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+def _matrix(t: torch.Tensor, cols: int) -> torch.Tensor:
+    """t.reshape(-1, cols) without the call where t has that shape already. With one row or one column the call stays: it
+    gives such an axis the pitch of a dense matrix, whatever the tensor's own says."""
+    if t.dim() == 2 and t.shape[1] == cols and cols > 1 and t.shape[0] > 1:
+        return t
+    return t.reshape(-1, cols)
+
+
+def _int16_vector(t: torch.Tensor, name: str) -> torch.Tensor:
+    """A parameter vector as the kernels read it: contiguous int16 on the GPU."""
+    _dev(t, name)
+    return t if t.dtype == torch.int16 and t.is_contiguous() else t.to(torch.int16).contiguous()
 
 
 def _rows2d(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -67,7 +83,7 @@ def _rows2d(t: torch.Tensor, name: str) -> torch.Tensor:
     _dev(t, name)
     if t.dim() < 1:
         raise ValueError(f'{name}: need at least one axis.')
-    t2 = t.reshape(-1, t.shape[-1])
+    t2 = _matrix(t, int(t.shape[-1]))
     if t2.stride(-1) != 1 and t2.shape[-1] > 1:
         t2 = t2.contiguous()
     return t2
@@ -244,7 +260,7 @@ def dense(x: torch.Tensor, p: PackedDense, rounding='floor', relu: bool = False,
     ok = _kind(out_kind)
     if out is None:
         out = torch.empty(tuple(x.shape[:-1]) + (p.N,), dtype=_KIND_TORCH[ok], device=x.device)
-    y2 = out.reshape(-1, p.N)
+    y2 = _matrix(out, p.N)
     if p.wt_lo is not None:
         if x2.dtype != torch.int16:
             raise RuntimeError('unsupported int8 x int16 precision mix for AIE implementations; no implementation variant '
@@ -348,8 +364,8 @@ def layernorm(x: torch.Tensor, gamma_q7: torch.Tensor, beta_q15: torch.Tensor, o
     if x2.dtype != torch.int8:
         raise NotImplementedError('integer LayerNorm needs signed 8-bit input and output')
     cols = int(x2.shape[1])
-    g = _dev(gamma_q7, 'gamma').to(torch.int16).contiguous()
-    b = _dev(beta_q15, 'beta').to(torch.int16).contiguous()
+    g = _int16_vector(gamma_q7, 'gamma')
+    b = _int16_vector(beta_q15, 'beta')
     if g.numel() != cols or b.numel() != cols:
         raise ValueError(f'LayerNorm parameter length does not match full_inner={cols}.')
     if out is None:
@@ -368,8 +384,8 @@ def add_layernorm(a: torch.Tensor, b: torch.Tensor, gamma_q7: torch.Tensor, beta
     a2 = _rows2d(a, 'a').contiguous()
     b2 = _rows2d(b, 'b').contiguous()
     cols = int(a2.shape[1])
-    g = _dev(gamma_q7, 'gamma').to(torch.int16).contiguous()
-    bt = _dev(beta_q15, 'beta').to(torch.int16).contiguous()
+    g = _int16_vector(gamma_q7, 'gamma')
+    bt = _int16_vector(beta_q15, 'beta')
     if g.numel() != cols or bt.numel() != cols:
         raise ValueError(f'LayerNorm parameter length does not match full_inner={cols}.')
     if out is None:
@@ -423,8 +439,8 @@ def dense_add_layernorm(x: torch.Tensor, p: PackedDense, residual: Optional[torc
         if residual.dtype != torch.int8 or tuple(residual.shape) != tuple(x.shape[:-1]) + (p.N,):
             raise ValueError('dense_add_layernorm: the residual must be an int8 tensor of the output shape')
         r2 = _pitched_rows(residual, 'residual')  # a window of a wider tensor is read where it lies
-    g = _dev(gamma_q7, 'gamma').to(torch.int16).contiguous()
-    bt = _dev(beta_q15, 'beta').to(torch.int16).contiguous()
+    g = _int16_vector(gamma_q7, 'gamma')
+    bt = _int16_vector(beta_q15, 'beta')
     if g.numel() != p.N or bt.numel() != p.N:
         raise ValueError(f'LayerNorm parameter length does not match full_inner={p.N}.')
     L = _lib.load()
@@ -581,8 +597,8 @@ def mlp_add_layernorm(x: torch.Tensor, layers: Sequence[MlpLayerSpec], residual:
         if residual.dtype != torch.int8 or tuple(residual.shape) != tuple(x.shape[:-1]) + (N,):
             raise ValueError('mlp_add_layernorm: the residual must be an int8 tensor of the output shape')
         r2 = _pitched_rows(residual, 'residual')  # a window of a wider tensor is read where it lies
-    g = _dev(gamma_q7, 'gamma').to(torch.int16).contiguous()
-    bt = _dev(beta_q15, 'beta').to(torch.int16).contiguous()
+    g = _int16_vector(gamma_q7, 'gamma')
+    bt = _int16_vector(beta_q15, 'beta')
     if g.numel() != N or bt.numel() != N:
         raise ValueError(f'LayerNorm parameter length does not match full_inner={N}.')
     if out is None:
@@ -641,13 +657,12 @@ def _attention(entry: str, q, k, v, logit_shift, logit_rounding, softmax, out_sh
         raise ValueError('attention: out must be int8 of shape [..., sq, d] with a contiguous last axis')
 
     def strides3(t):  # (batch, head, row) byte strides with missing leading axes as 0
-        st = [0] * (4 - t.dim()) + [int(x) for x in t.stride()]
-        return st[0], st[1], st[2]
+        return ((0,) * (4 - t.dim()) + t.stride())[:3]
 
     batch = int(lead[0]) if len(lead) >= 1 else 1
     heads = int(lead[1]) if len(lead) == 2 else 1
     if len(lead) == 1:  # [batch, s, d]: one head
-        flat = [(int(t.stride(0)), 0, int(t.stride(1))) for t in (q, k, v, out)]
+        flat = [(t.stride(0), 0, t.stride(1)) for t in (q, k, v, out)]
     else:
         flat = [strides3(t) for t in (q, k, v, out)]
     arr = (ctypes.c_int64 * 12)(*[x for trip in flat for x in trip])
@@ -735,7 +750,7 @@ def dense_float(x: torch.Tensor, p: PackedDenseFloat, relu: bool = False, out: O
     M = int(x2.shape[0])
     if out is None:
         out = torch.empty(tuple(x.shape[:-1]) + (p.N,), dtype=x.dtype, device=x.device)
-    y2 = out.reshape(-1, p.N)
+    y2 = _matrix(out, p.N)
     check(_lib.load().a4g_dense_f(_ptr(x2), fmt, 0, x2.stride(0) if M > 0 else p.K, _ptr(p.wt), p.ldwt, _ptr(p.bias),
                                   int(bool(relu)), _ptr(y2), y2.stride(0) if M > 0 else p.N, M, p.N, p.K, _stream()))
     return out
