@@ -394,8 +394,8 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
 }
 
 // Fitted to measurements (38 shapes of 1 to 8192 rows, 48 to 5000 inputs, 10 to 4096 outputs in every format): a launch of form f
-// takes start[f] us, plus tile[f] us for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus half a
-// microsecond for every workgroup of a CU after its first; the tiled kernels take other_start us plus other_tile us for every K
+// takes start[f] us, plus tile[f] us for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus `more` us
+// for every workgroup of a CU after its first; the tiled kernels take other_start us plus other_tile us for every K
 // tile, times the share of the chip that their 128 x 128 tiles need if that is more than all of it.
 // Measured, this kernel / the tiled ones, us: 16 x 4096 -> 4096 int8 5.4 / 22.3, int16 7.5 / 51, bfloat16 6.7 / 38, float32
 // 14 / 235, fp8 4.6 / 24; 128 x 3072 -> 768 int8 5.7 / 18.7; 128 x 768 -> 768 int8 4.6 / 7.7; 1024 x 768 -> 768 int8 6.9 / 7.8;
@@ -403,14 +403,15 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
 struct FewCosts {
     float start[4], tile[4];
     float other_start, other_tile;
+    float more;
 };
 static constexpr FewCosts FEW_COSTS[] = {
-    /* FEW_I8     */ {{3.9f, 4.1f, 4.0f, 6.8f}, {0.055f, 0.070f, 0.090f, 0.25f}, 6.0f, 0.50f},
-    /* FEW_I16X8  */ {{5.0f, 5.4f, 5.1f, 9.3f}, {0.080f, 0.100f, 0.160f, 0.52f}, 6.5f, 1.40f},
-    /* FEW_I16X16 */ {{5.8f, 6.4f, 6.2f, 0.0f}, {0.120f, 0.140f, 0.270f, 0.00f}, 6.5f, 1.45f},
-    /* FEW_BF16   */ {{3.5f, 3.6f, 3.5f, 4.9f}, {0.050f, 0.060f, 0.100f, 0.20f}, 5.5f, 0.51f},
-    /* FEW_F32    */ {{3.5f, 3.7f, 3.9f, 5.7f}, {0.080f, 0.104f, 0.190f, 0.50f}, 5.5f, 1.80f},
-    /* FEW_FP8    */ {{3.5f, 3.6f, 3.5f, 5.5f}, {0.036f, 0.050f, 0.088f, 0.20f}, 9.7f, 0.46f},
+    /* FEW_I8     */ {{3.9f, 4.1f, 4.0f, 6.8f}, {0.055f, 0.070f, 0.090f, 0.25f}, 6.0f, 0.50f, 0.5f},
+    /* FEW_I16X8  */ {{5.0f, 5.4f, 5.1f, 9.3f}, {0.080f, 0.100f, 0.160f, 0.52f}, 5.2f, 0.82f, 1.1f},
+    /* FEW_I16X16 */ {{5.8f, 6.4f, 6.2f, 0.0f}, {0.120f, 0.140f, 0.270f, 0.00f}, 7.2f, 1.17f, 2.0f},
+    /* FEW_BF16   */ {{3.5f, 3.6f, 3.5f, 4.9f}, {0.050f, 0.060f, 0.100f, 0.20f}, 5.5f, 0.51f, 0.5f},
+    /* FEW_F32    */ {{3.5f, 3.7f, 3.9f, 5.7f}, {0.080f, 0.104f, 0.190f, 0.50f}, 5.5f, 1.80f, 0.5f},
+    /* FEW_FP8    */ {{3.5f, 3.6f, 3.5f, 5.5f}, {0.036f, 0.050f, 0.088f, 0.20f}, 9.7f, 0.46f, 0.5f},
 };
 
 static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {
@@ -422,7 +423,7 @@ static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {
         const float rows = static_cast<float>((g.M + FEW_FORMS[f].tm * 16 - 1) / (FEW_FORMS[f].tm * 16));
         const float cols = static_cast<float>((g.N + FEW_FORMS[f].tn * 16 - 1) / (FEW_FORMS[f].tn * 16));
         const float per_cu = std::max(1.f, rows * cols * batch / 256.f);
-        const float t = c.start[f] + per_cu * ktiles * c.tile[f] + (per_cu - 1.f) * 0.5f;
+        const float t = c.start[f] + per_cu * ktiles * c.tile[f] + (per_cu - 1.f) * c.more;
         if (t < *us) {
             *us = t;
             best = f;

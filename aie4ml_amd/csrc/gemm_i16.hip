@@ -22,12 +22,12 @@
 
 namespace a4g {
 
-// LDS of the tiled kernels below: one stage of either is 30720 bytes (K step 64, rows padded to 80 bytes), which
-// the output image reuses. A reduction that fits one K tile takes a single stage, so more workgroups share a CU.
-constexpr int TILED16_STAGE_BYTES = 30720;
-static inline size_t tiled16_lds_bytes(int64_t K, int tile_rows) {
-    const size_t stages = static_cast<size_t>(K > 64 ? 2 : 1) * TILED16_STAGE_BYTES;
-    const size_t image = static_cast<size_t>(tile_rows) * (128 * 2 + 16);  // 128 two-byte outputs per row and its padding
+// LDS of the tiled kernels below: a stage holds so many rows of both operands' byte planes (K step 64, rows padded to 80
+// bytes); the output image reuses it. A reduction that fits one K tile takes a single stage, so more workgroups share a CU.
+constexpr int tiled16_stage_bytes(int plane_rows) { return plane_rows * 80; }
+static inline size_t tiled16_lds_bytes(int64_t K, int plane_rows, int tile_rows, int tile_cols) {
+    const size_t stages = static_cast<size_t>(K > 64 ? 2 : 1) * tiled16_stage_bytes(plane_rows);
+    const size_t image = static_cast<size_t>(tile_rows) * (tile_cols * 2 + 16);  // two-byte outputs of a row and its padding
     return stages > image ? stages : image;
 }
 
@@ -47,8 +47,8 @@ struct Gemm16Args {
     int trans_a;   // RAGGED kernels: A is stored transposed, [K][lda]
 };
 
-// 128 x 128 output tile, K step 64, 4 waves (2 x 2) of 64 x 64, double-buffered LDS holding the two byte
-// planes of A and the weight tile. Requires K % 8 == 0 and 16-byte aligned rows of A and Wt.
+// 128 x BN output tile, K step 64, 4 waves (2 x 2) of 64 x BN / 2, double-buffered LDS holding the two byte
+// planes of A and the weight tile.
 __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
     const int obytes = (g.out_kind == A4G_I16 || g.out_kind == A4G_U16) ? 2 : 1;
     g.A += b * g.stride_a;
@@ -57,13 +57,20 @@ __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
     g.Y = static_cast<int8_t*>(g.Y) + b * g.stride_y * obytes;
 }
 
-// RAGGED: K need not be a multiple of 16 nor A's rows 16-byte aligned (the packed weights always are, zero padded).
-template <bool RAGGED>
-__global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
-    constexpr int BM = 128, BN = 128, BK = 64, PITCH = BK + 16;
+// ROWS: how A is read. 0: rows 16-byte aligned, K a multiple of 16. 1: any address, any K of 8 or more (one unaligned load
+// per chunk, the chunk that crosses a row's end moved into place as it is staged). 2: stored transposed, shorter, or a pitch
+// beyond 32-bit offsets (loads in branches). The packed weights are aligned and zero padded to 16 in every form.
+// A K tile is 0.2 us of matrix work and a load takes 1 us and more, so forms 0 and 1 have two K tiles on their way in
+// registers beside the one in LDS, fetched through buffer descriptors (past K or past the last row reads as zero: no load
+// stands in a branch, so every wait counts exactly). Rate by size in the comment at the launch.
+template <int ROWS, int BN>
+__global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm16Args g) {
+    constexpr bool RAGGED = ROWS == 2;
+    constexpr int SETS = RAGGED ? 1 : 2;
+    constexpr int BM = 128, BK = 64, PITCH = BK + 16, TN = BN / 64, LB = BN / 64;  // a wave: 64 rows, BN / 2 columns
     select_problem(g, blockIdx.y);
     constexpr int PLANE = BM * PITCH, STAGE = 2 * PLANE + BN * PITCH;
-    static_assert(STAGE == TILED16_STAGE_BYTES, "the launch sizes the LDS");
+    static_assert(STAGE == tiled16_stage_bytes(2 * BM + BN), "the launch sizes the LDS");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];  // two stages, or one when K fits a single tile
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -97,34 +104,53 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
     fetch_col_params<BN, true>(eg, here, tid, col_add, col_shift);
 
     // staging: A tile = 128 rows x 8 chunks of 8 int16 (4 per thread), W tile = 128 rows x 4 chunks of 16 int8 (2 per thread)
-    v4i ra[4], rb[2];
-    auto load_tile = [&](int k0) {
+    v4i stage_a[SETS][4], stage_b[SETS][LB];
+    const int lda2 = static_cast<int>(g.lda) * 2, ldwt = static_cast<int>(g.ldwt);
+    const int64_t range_a = (static_cast<int64_t>(g.M - 1 - m0) * g.lda + g.K) * 2;
+    const int64_t range_b = static_cast<int64_t>(g.N - 1 - n0) * g.ldwt + (g.K + 15) / 16 * 16;
+    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int16_t*>(g.A + static_cast<int64_t>(m0) * g.lda), 0, static_cast<int>(range_a < 0x7fffffff ? range_a : 0x7fffffff), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(g.Wt + static_cast<int64_t>(n0) * g.ldwt), 0, static_cast<int>(range_b < 0x7fffffff ? range_b : 0x7fffffff), 0x00020000);
+    auto load_tile = [&](int set, int k0) __attribute__((always_inline)) {
+        v4i (&ra)[4] = stage_a[set];
+        v4i (&rb)[LB] = stage_b[set];
+        if constexpr (!RAGGED) {
+            constexpr unsigned NOWHERE = 0x80000000u;  // beyond both descriptors, whatever is added: reads as zero
+            const int ka = k0 + (tid & 7) * 8, kb = k0 + (tid & 3) * 16;
+            const int at = ROWS == 1 ? min(ka, g.K - 8) : ka;
+            const unsigned off_a = ka < g.K ? static_cast<unsigned>((tid >> 3) * lda2 + at * 2) : NOWHERE;
+            const unsigned off_b = kb < g.K ? static_cast<unsigned>((tid >> 2) * ldwt + kb) : NOWHERE;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ra[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off_a + i * 32 * lda2, 0, 0));
+#pragma unroll
+            for (int i = 0; i < LB; ++i) rb[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, off_b + i * 64 * ldwt, 0, 0));
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
             const int gm = min(m0 + row, g.M - 1);
-            if constexpr (RAGGED)
-                ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
-                                  : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                      (g.K - (k0 + kc)) * 2, g.K * 2);
-            else
-                ra[i] = (k0 + kc < g.K) ? *reinterpret_cast<const v4i*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc)
-                                        : v4i{0, 0, 0, 0};
+            ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
+                              : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
+                                                  (g.K - (k0 + kc)) * 2, g.K * 2);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < LB; ++i) {
             const int c = tid + i * 256, row = c >> 2, kc = (c & 3) * 16;
             const int gn = min(n0 + row, g.N - 1);
             rb[i] = (k0 + kc < g.K) ? *reinterpret_cast<const v4i*>(g.Wt + static_cast<int64_t>(gn) * g.ldwt + k0 + kc)
                                     : v4i{0, 0, 0, 0};
         }
     };
-    auto store_tile = [&](int buf, int k0) {
+    auto store_tile = [&](int set, int buf, int k0) __attribute__((always_inline)) {
+        v4i (&ra)[4] = stage_a[set];
+        v4i (&rb)[LB] = stage_b[set];
         int8_t* st = smem + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
-            if (RAGGED && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
+            if (ROWS != 0 && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             // eight int16 in four dwords -> their eight high bytes and eight low bytes
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             v2i hi = {static_cast<int>(__builtin_amdgcn_perm(w1, w0, 0x07050301u)), static_cast<int>(__builtin_amdgcn_perm(w3, w2, 0x07050301u))};
@@ -134,64 +160,106 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i8_kernel(Gemm16Args g) {
             *reinterpret_cast<v2i*>(st + PLANE + row * PITCH + kc) = lo;
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < LB; ++i) {
             const int c = tid + i * 256, row = c >> 2, kc = (c & 3) * 16;
             *reinterpret_cast<v4i*>(st + 2 * PLANE + row * PITCH + kc) = rb[i];
         }
     };
 
-    v16i acc_hi[2][2], acc_lo[2][2];
+    v16i acc_hi[2][TN], acc_lo[2][TN];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc_hi[i][j][r] = acc_lo[i][j][r] = 0;
 
     const int frow = lane & 31, fk = (lane >> 5) * 16;
-    const int a_off = (wm * 64 + frow) * PITCH + fk, b_off = 2 * PLANE + (wn * 64 + frow) * PITCH + fk;
+    const int a_off = (wm * 64 + frow) * PITCH + fk, b_off = 2 * PLANE + (wn * (BN / 2) + frow) * PITCH + fk;
     const int ktiles = (g.K + BK - 1) / BK;
-    load_tile(0);
+    load_tile(0, 0);
+    if constexpr (SETS == 2) load_tile(1, BK);
     const int round_path = park_col_params<BN>(eg, cp, tid, col_add, col_shift);  // contains barriers
-    store_tile(0, 0);
+    store_tile(0, 0, 0);
+    if constexpr (SETS == 2) load_tile(0, 2 * BK);
     __syncthreads();
-    for (int kt = 0; kt < ktiles; ++kt) {
-        const int8_t* st = smem + (kt & 1) * STAGE;
-        if (kt + 1 < ktiles) load_tile((kt + 1) * BK);
+    // one half of a K tile: 32 elements
+    auto half = [&](const int8_t* st, int kk) __attribute__((always_inline)) {
+        v4i ah[2], al[2], bf[TN];
 #pragma unroll
-        for (int kk = 0; kk < BK / 32; ++kk) {
-            v4i ah[2], al[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                ah[i] = *reinterpret_cast<const v4i*>(st + a_off + i * 32 * PITCH + kk * 32);
-                al[i] = *reinterpret_cast<const v4i*>(st + PLANE + a_off + i * 32 * PITCH + kk * 32);
-                bf[i] = *reinterpret_cast<const v4i*>(st + b_off + i * 32 * PITCH + kk * 32);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    // operands swapped: lanes run over rows m, accumulator registers over columns n
-                    acc_hi[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], ah[i], acc_hi[i][j], 0, 0, 0);
-                    acc_lo[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], al[i], acc_lo[i][j], 0, 0, 0);
-                }
+        for (int i = 0; i < 2; ++i) {
+            ah[i] = *reinterpret_cast<const v4i*>(st + a_off + i * 32 * PITCH + kk * 32);
+            al[i] = *reinterpret_cast<const v4i*>(st + PLANE + a_off + i * 32 * PITCH + kk * 32);
         }
-        if (kt + 1 < ktiles) store_tile((kt + 1) & 1, (kt + 1) * BK);
-        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bf[j] = *reinterpret_cast<const v4i*>(st + b_off + j * 32 * PITCH + kk * 32);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                // operands swapped: lanes run over rows m, accumulator registers over columns n
+                acc_hi[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], ah[i], acc_hi[i][j], 0, 0, 0);
+                acc_lo[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], al[i], acc_lo[i][j], 0, 0, 0);
+            }
+    };
+    // `set` holds K tile kt + 1, which goes to the other LDS stage (its readers passed the last barrier) and makes room for
+    // tile kt + 1 + SETS; the loads behind RAGGED's branches are issued ahead of the matrix work instead
+    auto tile = [&](int kt, int set) __attribute__((always_inline)) {
+        const int8_t* st = smem + (kt & 1) * STAGE;
+        const bool more = kt + 1 < ktiles;
+        if (RAGGED && more) load_tile(0, (kt + 1) * BK);
+        half(st, 0);
+        if (!RAGGED) {
+            __builtin_amdgcn_sched_barrier(0);  // (a half's fragments at a time: both halves' would not fit the registers)
+            if (more) store_tile(set, (kt + 1) & 1, (kt + 1) * BK);
+            load_tile(set, (kt + 1 + SETS) * BK);
+        }
+        half(st, 1);
+        if (RAGGED && more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkmcnt0();  // (a __syncthreads may also wait for the loads)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (RAGGED) {
+        for (int kt = 0; kt < ktiles; ++kt) tile(kt, 0);
+    } else {
+        for (int kt = 0; kt + 1 < ktiles; kt += 2) {  // (with an exit in its middle it would keep the accumulators twice)
+            tile(kt, 1);
+            tile(kt + 1, 0);
+        }
+        if (ktiles & 1) tile(ktiles - 1, 1);
     }
+    __syncthreads();
 
     // epilogue: lane owns row lane%32 of each block and, per register quad q, columns 8q + 4*(lane/32) .. +3
     // a.w = 256 * sum(hi.w) + sum((lo - 128).w) + 128 * sum(w): the last term is in the column's addend. The tile
     // leaves through the epilogue of the int8 kernels (the stages are dead: the loop ended on a barrier).
-    v16i sum[2][2];
+    v16i sum[2][TN];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 sum[i][j][r] = static_cast<int>((static_cast<unsigned>(acc_hi[i][j][r]) << 8) + static_cast<unsigned>(acc_lo[i][j][r]));
-    epilogue_store<BM, BN, 64, 64, 256>(eg, here, sum, smem, cp, round_path, wm, wn, lane, tid);
+    epilogue_store<BM, BN, 64, BN / 2, 256>(eg, here, sum, smem, cp, round_path, wm, wn, lane, tid);
+}
+
+template <int ROWS, int BN>
+static void launch_i16i8_form(const Gemm16Args& g, unsigned batch, hipStream_t stream) {
+    const int64_t tiles = (static_cast<int64_t>(g.M) + 127) / 128 * ((g.N + BN - 1) / BN);
+    const dim3 grid(static_cast<unsigned>(grid_for_tiles(tiles)), batch);  // whole ranges for the 8 XCDs
+    gemm_i16i8_kernel<ROWS, BN><<<grid, 256, tiled16_lds_bytes(g.K, 256 + BN, 128, BN), stream>>>(g);
+}
+
+// `aligned`: A stored row by row, rows 16-byte aligned, K a multiple of 16. The forms that fetch through descriptors hold a
+// tile's 128 rows within 30-bit offsets.
+static void launch_tiled_i16i8(const Gemm16Args& g, unsigned batch, bool aligned, hipStream_t stream) {
+    const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23);
+    if (near && aligned) launch_i16i8_form<0, 64>(g, batch, stream);
+    else if (near && !g.trans_a && g.K >= 8) launch_i16i8_form<1, 64>(g, batch, stream);
+    else launch_i16i8_form<2, 128>(g, batch, stream);
 }
 
 // Any K / alignment: one thread per output element.
@@ -407,12 +475,15 @@ __device__ __forceinline__ void select_problem(Gemm16x16Args& g, int b) {
     g.Y = static_cast<int8_t*>(g.Y) + b * g.stride_y * obytes;
 }
 
-template <bool RAGGED>
+// ROWS and the two K tiles on their way in registers: as in gemm_i16i8_kernel.
+template <int ROWS>
 __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
+    constexpr bool RAGGED = ROWS == 2;
+    constexpr int SETS = RAGGED ? 1 : 2;
     constexpr int BM = 64, BN = 128, BK = 64, PITCH = BK + 16;
     select_problem(g, blockIdx.y);
     constexpr int APLANE = BM * PITCH, WPLANE = BN * PITCH, STAGE = 2 * APLANE + 2 * WPLANE;
-    static_assert(STAGE == TILED16_STAGE_BYTES, "the launch sizes the LDS");
+    static_assert(STAGE == tiled16_stage_bytes(2 * (BM + BN)), "the launch sizes the LDS");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];  // two stages, or one when K fits a single tile
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -440,19 +511,42 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
     }
 
     // staging: A tile = 64 rows x 8 chunks of 8 int16 (2 per thread); each W plane = 128 rows x 4 chunks (2 per thread)
-    v4i ra[2], rh[2], rl[2];
-    auto load_tile = [&](int k0) {
+    v4i stage_a[SETS][2], stage_h[SETS][2], stage_l[SETS][2];
+    const int lda2 = static_cast<int>(g.lda) * 2, ldwt = static_cast<int>(g.ldwt);
+    const int64_t range_a = (static_cast<int64_t>(g.M - 1 - m0) * g.lda + g.K) * 2;
+    const int64_t range_b = static_cast<int64_t>(g.N - 1 - n0) * g.ldwt + (g.K + 15) / 16 * 16;
+    const int records_b = static_cast<int>(range_b < 0x7fffffff ? range_b : 0x7fffffff);
+    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int16_t*>(g.A + static_cast<int64_t>(m0) * g.lda), 0, static_cast<int>(range_a < 0x7fffffff ? range_a : 0x7fffffff), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_h =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(g.Wh + static_cast<int64_t>(n0) * g.ldwt), 0, records_b, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_l =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(g.Wl + static_cast<int64_t>(n0) * g.ldwt), 0, records_b, 0x00020000);
+    auto load_tile = [&](int set, int k0) __attribute__((always_inline)) {
+        v4i (&ra)[2] = stage_a[set];
+        v4i (&rh)[2] = stage_h[set];
+        v4i (&rl)[2] = stage_l[set];
+        if constexpr (!RAGGED) {
+            constexpr unsigned NOWHERE = 0x80000000u;  // beyond the descriptors, whatever is added: reads as zero
+            const int ka = k0 + (tid & 7) * 8, kb = k0 + (tid & 3) * 16;
+            const int at = ROWS == 1 ? min(ka, g.K - 8) : ka;
+            const unsigned off_a = ka < g.K ? static_cast<unsigned>((tid >> 3) * lda2 + at * 2) : NOWHERE;
+            const unsigned off_b = kb < g.K ? static_cast<unsigned>((tid >> 2) * ldwt + kb) : NOWHERE;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                ra[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off_a + i * 32 * lda2, 0, 0));
+                rh[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_h, off_b + i * 64 * ldwt, 0, 0));
+                rl[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_l, off_b + i * 64 * ldwt, 0, 0));
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
             const int gm = min(m0 + row, g.M - 1);
-            if constexpr (RAGGED)
-                ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
-                                  : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                      (g.K - (k0 + kc)) * 2, g.K * 2);
-            else
-                ra[i] = (k0 + kc < g.K) ? *reinterpret_cast<const v4i*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc)
-                                        : v4i{0, 0, 0, 0};
+            ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
+                              : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
+                                                  (g.K - (k0 + kc)) * 2, g.K * 2);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -464,15 +558,18 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
             rl[i] = in ? *reinterpret_cast<const v4i*>(g.Wl + static_cast<int64_t>(gn) * g.ldwt + k0 + kc) : v4i{0, 0, 0, 0};
         }
     };
-    auto store_tile = [&](int buf, int k0) {
+    auto store_tile = [&](int set, int buf, int k0) __attribute__((always_inline)) {
+        v4i (&ra)[2] = stage_a[set];
+        v4i (&rh)[2] = stage_h[set];
+        v4i (&rl)[2] = stage_l[set];
         int8_t* st = smem + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
-            if (RAGGED && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
+            if (ROWS != 0 && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             // beyond K both planes are zero, so the row sums stay exact: the low bytes are biased where k < K only
-            const int live = min(max(g.K - (k0 + kc), 0), 8);  // elements of this chunk below K (0 or 8 unless RAGGED)
+            const int live = min(max(g.K - (k0 + kc), 0), 8);  // elements of this chunk below K (0 or 8 where K is in whole chunks)
             const unsigned flip0 = live >= 4 ? 0x80808080u : (0x80808080u & ((1u << (8 * live)) - 1u));
             const unsigned flip1 = live >= 8 ? 0x80808080u : (live > 4 ? (0x80808080u & ((1u << (8 * (live - 4))) - 1u)) : 0u);
             v2i hi = {static_cast<int>(__builtin_amdgcn_perm(w1, w0, 0x07050301u)), static_cast<int>(__builtin_amdgcn_perm(w3, w2, 0x07050301u))};
@@ -499,38 +596,61 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
     const int frow = lane & 31, fk = (lane >> 5) * 16;
     const int a_off = (wm * 32 + frow) * PITCH + fk, b_off = 2 * APLANE + (wn * 64 + frow) * PITCH + fk;
     const int ktiles = (g.K + BK - 1) / BK;
-    load_tile(0);
-    store_tile(0, 0);
+    load_tile(0, 0);
+    if constexpr (SETS == 2) load_tile(1, BK);
+    store_tile(0, 0, 0);
+    if constexpr (SETS == 2) load_tile(0, 2 * BK);
     __syncthreads();
-    for (int kt = 0; kt < ktiles; ++kt) {
-        const int8_t* st = smem + (kt & 1) * STAGE;
-        if (kt + 1 < ktiles) load_tile((kt + 1) * BK);
+    // one half of a K tile: 32 elements
+    auto half = [&](const int8_t* st, int kk) __attribute__((always_inline)) {
+        const v4i ah = *reinterpret_cast<const v4i*>(st + a_off + kk * 32);
+        const v4i al = *reinterpret_cast<const v4i*>(st + APLANE + a_off + kk * 32);
+        v4i bh[2], bl[2];
 #pragma unroll
-        for (int kk = 0; kk < BK / 32; ++kk) {
-            const v4i ah = *reinterpret_cast<const v4i*>(st + a_off + kk * 32);
-            const v4i al = *reinterpret_cast<const v4i*>(st + APLANE + a_off + kk * 32);
-            v4i bh[2], bl[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                bh[j] = *reinterpret_cast<const v4i*>(st + b_off + j * 32 * PITCH + kk * 32);
-                bl[j] = *reinterpret_cast<const v4i*>(st + WPLANE + b_off + j * 32 * PITCH + kk * 32);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                rs_hi = __builtin_amdgcn_sdot4(ah[t], 0x01010101, rs_hi, false);
-                rs_lo = __builtin_amdgcn_sdot4(al[t], 0x01010101, rs_lo, false);
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                acc_hh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bh[j], ah, acc_hh[j], 0, 0, 0);
-                acc_hl[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bl[j], ah, acc_hl[j], 0, 0, 0);
-                acc_lh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bh[j], al, acc_lh[j], 0, 0, 0);
-                acc_ll[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bl[j], al, acc_ll[j], 0, 0, 0);
-            }
+        for (int j = 0; j < 2; ++j) {
+            bh[j] = *reinterpret_cast<const v4i*>(st + b_off + j * 32 * PITCH + kk * 32);
+            bl[j] = *reinterpret_cast<const v4i*>(st + WPLANE + b_off + j * 32 * PITCH + kk * 32);
         }
-        if (kt + 1 < ktiles) store_tile((kt + 1) & 1, (kt + 1) * BK);
-        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            rs_hi = __builtin_amdgcn_sdot4(ah[t], 0x01010101, rs_hi, false);
+            rs_lo = __builtin_amdgcn_sdot4(al[t], 0x01010101, rs_lo, false);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            acc_hh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bh[j], ah, acc_hh[j], 0, 0, 0);
+            acc_hl[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bl[j], ah, acc_hl[j], 0, 0, 0);
+            acc_lh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bh[j], al, acc_lh[j], 0, 0, 0);
+            acc_ll[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bl[j], al, acc_ll[j], 0, 0, 0);
+        }
+    };
+    auto tile = [&](int kt, int set) __attribute__((always_inline)) {  // as in gemm_i16i8_kernel
+        const int8_t* st = smem + (kt & 1) * STAGE;
+        const bool more = kt + 1 < ktiles;
+        if (RAGGED && more) load_tile(0, (kt + 1) * BK);
+        half(st, 0);
+        if (!RAGGED) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (more) store_tile(set, (kt + 1) & 1, (kt + 1) * BK);
+            load_tile(set, (kt + 1 + SETS) * BK);
+        }
+        half(st, 1);
+        if (RAGGED && more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkmcnt0();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (RAGGED) {
+        for (int kt = 0; kt < ktiles; ++kt) tile(kt, 0);
+    } else {
+        for (int kt = 0; kt + 1 < ktiles; kt += 2) {
+            tile(kt, 1);
+            tile(kt + 1, 0);
+        }
+        if (ktiles & 1) tile(ktiles - 1, 1);
     }
+    __syncthreads();
     // the other half of the row's k range sits in lane ^ 32
     rs_hi += __shfl_xor(rs_hi, 32);
     rs_lo += __shfl_xor(rs_lo, 32);
@@ -576,6 +696,15 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
     TileCoord here = tc;
     here.batch = 0;  // select_problem has already moved the pointers to this problem
     store_tile_image<BM, BN, 256>(img, here, smem, obytes, tid);
+}
+
+// `aligned` and the limit on the pitches as in launch_tiled_i16i8.
+static void launch_tiled_i16i16(const Gemm16x16Args& g, dim3 grid, bool aligned, hipStream_t stream) {
+    const size_t lds = tiled16_lds_bytes(g.K, 384, 64, 128);
+    const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23);
+    if (near && aligned) gemm_i16i16_kernel<0><<<grid, 256, lds, stream>>>(g);
+    else if (near && !g.trans_a && g.K >= 8) gemm_i16i16_kernel<1><<<grid, 256, lds, stream>>>(g);
+    else gemm_i16i16_kernel<2><<<grid, 256, lds, stream>>>(g);
 }
 
 // Any K / alignment: one thread per output element, straight from the planes (w = 256 wh + (wl ^ 0x80 as unsigned)).
@@ -731,14 +860,8 @@ extern "C" int a4g_dense_i16(const int16_t* A, int trans_a, int64_t lda, const i
     A4G_REQUIRE(!trans_a || w_ok, A4G_ERR_UNSUPPORTED, "%s: a transposed left operand needs weights as a4g_pack_weights_i8 writes them", who);
     g.trans_a = trans_a != 0;
     if (w_ok) {
-        const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-        A4G_REQUIRE(tiles <= INT32_MAX, A4G_ERR_UNSUPPORTED, "%s: too many tiles", who);
-        const dim3 grid(static_cast<unsigned>(grid_for_tiles(tiles)), 1);  // whole ranges for the 8 XCDs
-        if (!trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A)) {
-            gemm_i16i8_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
-        } else {
-            gemm_i16i8_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
-        }
+        A4G_REQUIRE(((M + 127) / 128) * ((N + 127) / 128) <= INT32_MAX / 2, A4G_ERR_UNSUPPORTED, "%s: too many tiles", who);
+        launch_tiled_i16i8(g, 1, !trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A), stream);
     } else {
         const int grid = static_cast<int>(std::min<int64_t>((M * N + 255) / 256, 256 * 32));
         gemm_i16i8_generic_kernel<<<grid, 256, 0, stream>>>(g);
@@ -799,12 +922,7 @@ extern "C" int a4g_dense_i16x16(const int16_t* A, int trans_a, int64_t lda, cons
     if (w_ok) {
         const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128);
         A4G_REQUIRE(tiles <= INT32_MAX, A4G_ERR_UNSUPPORTED, "%s: too many tiles", who);
-        const dim3 grid(static_cast<unsigned>(grid_for_tiles(tiles)), 1);
-        if (!trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A)) {
-            gemm_i16i16_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
-        } else {
-            gemm_i16i16_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
-        }
+        launch_tiled_i16i16(g, dim3(static_cast<unsigned>(grid_for_tiles(tiles)), 1), !trans_a && K % 16 == 0 && lda % 8 == 0 && aligned16(A), stream);
     } else {
         const int grid = static_cast<int>(std::min<int64_t>((M * N + 255) / 256, 256 * 32));
         gemm_i16i16_generic_kernel<<<grid, 256, 0, stream>>>(g);
@@ -870,12 +988,8 @@ extern "C" int a4g_matmul_i16(const int16_t* A, int trans_a, int64_t lda, int64_
             return check_hip(launch_rs_policy<I16x16Policy, 256, 256, 2, 4, true>(r, nb, stream), who);
         g.trans_a = trans_a != 0;
         const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128);
-        const dim3 grid(static_cast<unsigned>(grid_for_tiles(tiles)), nb);
-        if (tiled) {
-            gemm_i16i16_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
-        } else {  // the packed planes in the workspace are always aligned and zero padded; A is fetched as its rows allow
-            gemm_i16i16_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 64), stream>>>(g);
-        }
+        // (the packed planes in the workspace are always aligned and zero padded)
+        launch_tiled_i16i16(g, dim3(static_cast<unsigned>(grid_for_tiles(tiles)), nb), tiled, stream);
     } else {
         Gemm16Args g{};
         g.A = A; g.Wt = hi; g.colsum = colsum; g.bias = nullptr; g.shifts = nullptr; g.Y = C;
@@ -891,13 +1005,7 @@ extern "C" int a4g_matmul_i16(const int16_t* A, int trans_a, int64_t lda, int64_
         r.shift = shift; r.out_kind = out_kind; r.mode = round_mode;
         if (!trans_a && rs_i16i8_applicable(r, nb)) return check_hip(launch_rs_i16i8(r, nb, stream), who);
         g.trans_a = trans_a != 0;
-        const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-        const dim3 grid(static_cast<unsigned>(grid_for_tiles(tiles)), nb);
-        if (tiled) {
-            gemm_i16i8_kernel<false><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
-        } else {
-            gemm_i16i8_kernel<true><<<grid, 256, tiled16_lds_bytes(g.K, 128), stream>>>(g);
-        }
+        launch_tiled_i16i8(g, nb, tiled, stream);
     }
     return check_hip(hipGetLastError(), who);
 }

@@ -188,3 +188,20 @@ def test_dense_float_with_few_output_tiles(ops, oracle, fmt, M, K, N):
     for relu in (False, True):
         got = host(ops.dense_float(dev(A, fmt), p, relu=relu))
         check(got, oracle.dense_float(A, W, b, relu=relu, fmt=fmt), fmt, K, np.abs(A).astype(np.float64) @ np.abs(W) + np.abs(b))
+
+
+@pytest.mark.parametrize('fmt', ['bfloat16', 'float32'])
+@pytest.mark.parametrize('K', [32, 64, 96, 129, 200, 257, 320])
+def test_dense_float_with_two_k_tiles_ahead(ops, oracle, fmt, K):
+    """Enough output tiles for the tiled kernel, reductions of one to ten K tiles of 128 bytes, odd and even, whole and not,
+    rows aligned and at odd elements with NaN around them. Small integers: every order of summation gives the same bits."""
+    r = np.random.default_rng(K)
+    M, N = 8200, 330
+    A, W = (r.integers(-2, 3, sh).astype(np.float32) for sh in ((M, K), (K, N)))
+    t = {'bfloat16': torch.bfloat16, 'float32': torch.float32}[fmt]
+    wide = torch.full((M, K + 8), float('nan')).to(t)
+    wide[:, 1:K + 1] = torch.from_numpy(A).to(t)
+    p = ops.pack_dense_float(torch.from_numpy(W).to(t).cuda(), None)
+    want = torch.from_numpy(A @ W).to(t)
+    for x in (torch.from_numpy(A).to(t).cuda(), wide.cuda()[:, 1:K + 1]):
+        assert torch.equal(ops.dense_float(x, p).cpu(), want), tuple(x.stride())

@@ -1424,3 +1424,23 @@ def test_concat_places_parts_with_the_device_copy(ops, axis, dtype):
     np.testing.assert_array_equal(got.cpu().numpy(), np.concatenate(parts, axis=axis))
     with pytest.raises(ValueError, match='share dtype'):
         ops.concat([dev_parts[0], dev_parts[0][:, :1, :1]], axis)
+
+
+@pytest.mark.parametrize('K', [64, 129, 200, 255, 384, 520, 640])
+@pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
+def test_dense_with_two_k_tiles_ahead(ops, oracle, kind, K):
+    """Enough output tiles for the tiled kernels, reductions of one to five K tiles of 128 bytes (two to ten of 64 elements
+    of 16 bits, odd and even), whole and not, rows 16-byte aligned and at odd elements between extreme values; the last row
+    and column tiles are partial."""
+    r = rng(K + 11 * len(kind))
+    M, N = 8200, 330
+    adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
+    info = np.iinfo(adt)
+    W = r.integers(-32768, 32768, (K, N)).astype(np.int16) if kind == 'int16x16' else gauss8(r, 40, (K, N))
+    shift, out = (26, 'int16') if kind == 'int16x16' else (16, 'int16') if kind == 'int16x8' else (10, 'int8')
+    p = ops.pack_dense(dev(W), None, shift)
+    wide = np.where(np.arange(K + 16) % 2, info.max, info.min).astype(adt)[None].repeat(M, 0)
+    A = wide[:, 1:K + 1] = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+    want = oracle.dense(np.ascontiguousarray(A), W, None, np.array([shift]), 'conv_even', out=out)
+    for x in (dev(np.ascontiguousarray(A)), dev(wide)[:, 1:K + 1]):
+        assert np.array_equal(host(ops.dense(x, p, 'conv_even', out_kind=out)), want), tuple(x.stride())
