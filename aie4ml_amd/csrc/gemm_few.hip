@@ -153,6 +153,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(GemmArgs g, int tiles
 #pragma unroll
             for (int i = 0; i < LA; ++i)
                 if (at < ka) ra[slot][i] = chunk_in_place(ra[slot][i], ka - at, ka);
+            if constexpr (O::FLOAT) {  // what lies between K and the next chunk of a MatMul's operand is not its own: 0 * NaN
+                const int rem = kb - (kt * 128 + bchunk * 16);
+#pragma unroll
+                for (int j = 0; j < LB; ++j)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int v = rem - 4 * t;  // bytes of this dword that belong to K
+                        if (v <= 0) rb[slot][0][j][t] = 0;
+                        else if (v < 4) rb[slot][0][j][t] &= static_cast<int>((1u << (8 * v)) - 1u);
+                    }
+            }
         }
 #pragma unroll
         for (int i = 0; i < LA; ++i) {

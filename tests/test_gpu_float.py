@@ -205,3 +205,24 @@ def test_dense_float_with_two_k_tiles_ahead(ops, oracle, fmt, K):
     want = torch.from_numpy(A @ W).to(t)
     for x in (torch.from_numpy(A).to(t).cuda(), wide.cuda()[:, 1:K + 1]):
         assert torch.equal(ops.dense_float(x, p).cpu(), want), tuple(x.stride())
+
+
+@pytest.mark.parametrize('fmt', FORMATS)
+@pytest.mark.parametrize('K', [9, 33, 131, 300])
+def test_matmul_float_in_place_operand_with_nan_behind_its_rows(ops, fmt, K):
+    """A transposed right operand on 16-byte aligned rows whose pitch holds NaN past K: few output tiles, so the kernel
+    whose waves share K reads it where it lies. Small integers: every order of summation gives the same bits."""
+    from aie4ml_amd import _lib
+
+    r = np.random.default_rng(K)
+    M, N, t = 20, 37, TORCH_DT[fmt]
+    A, B = (r.integers(-1, 2, sh).astype(np.float32) for sh in ((M, K), (N, K)))
+    A[:, 16:] = 0  # sums up to 16: exact in every format
+    ld = -(-K // 16) * 16
+    wide = torch.full((N, ld), float('nan')).to(t)
+    wide[:, :K] = torch.from_numpy(B).to(t)
+    a, b = torch.from_numpy(A).to(t).cuda(), wide.cuda()
+    out = torch.empty((M, N), dtype=t, device='cuda')
+    _lib.check(_lib.load().a4g_matmul_f(ops._ptr(a), ops._float_format(a, 'a'), 0, K, M * K, ops._ptr(b), ld, N * ld, 1, ops._ptr(out), N,
+                                        M * N, 1, M, N, K, None, 0, ops._stream()))
+    assert torch.equal(out.float().cpu(), torch.from_numpy(A @ B.T))
