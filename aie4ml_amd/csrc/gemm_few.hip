@@ -8,6 +8,7 @@
 // floating-point sums get another order, as with any tiling.
 // Bound by the latency of the loads and by what a CU can draw from L2, not by the matrix unit.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "float_formats.hpp"
@@ -404,25 +405,27 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
     }
 }
 
-// Fitted to measurements (38 shapes of 1 to 8192 rows, 48 to 5000 inputs, 10 to 4096 outputs in every format): a launch of form f
+// Fitted to measurements (38 shapes of 1 to 8192 rows, 48 to 5000 inputs, 10 to 4096 outputs in every format, and a grid of 17 to 4096
+// rows, 32 to 2048 inputs, 64 to 2048 outputs: 1716 shapes in int8, 140 in each floating-point format): a launch of form f
 // takes start[f] us, plus tile[f] us for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus `more` us
 // for every workgroup of a CU after its first; the tiled kernels take other_start us plus other_tile us for every K
 // tile, times the share of the chip that their 128 x 128 tiles need if that is more than all of it.
 // Measured, this kernel / the tiled ones, us: 16 x 4096 -> 4096 int8 5.4 / 22.3, int16 7.5 / 51, bfloat16 6.7 / 38, float32
 // 14 / 235, fp8 4.6 / 24; 128 x 3072 -> 768 int8 5.7 / 18.7; 128 x 768 -> 768 int8 4.6 / 7.7; 1024 x 768 -> 768 int8 6.9 / 7.8;
-// 2048 x 768 -> 768 int8 10.1 / 9.6 (not taken); 512 x 4096 -> 4096 int8 21.5 / 26.4; 100 x 5000 -> 10 int8 5.7 / 34.
+// 2048 x 768 -> 768 int8 10.1 / 9.6 (not taken); 512 x 4096 -> 4096 int8 21.5 / 26.4; 100 x 5000 -> 10 int8 5.7 / 34;
+// 2048 x 256 -> 768 int8 9.4 / 7.3, 4096 x 64 -> 1536 bfloat16 21.0 / 9.0, 4096 x 256 -> 1536 fp8 20.7 / 13.4 (none of them taken).
 struct FewCosts {
     float start[4], tile[4];
     float other_start, other_tile;
     float more;
 };
 static constexpr FewCosts FEW_COSTS[] = {
-    /* FEW_I8     */ {{3.9f, 4.1f, 4.0f, 6.8f}, {0.055f, 0.070f, 0.090f, 0.25f}, 6.0f, 0.50f, 0.5f},
+    /* FEW_I8     */ {{3.9f, 4.1f, 4.0f, 6.8f}, {0.055f, 0.070f, 0.090f, 0.25f}, 6.0f, 0.50f, 0.8f},
     /* FEW_I16X8  */ {{5.0f, 5.4f, 5.1f, 9.3f}, {0.080f, 0.100f, 0.160f, 0.52f}, 5.2f, 0.82f, 1.1f},
     /* FEW_I16X16 */ {{5.8f, 6.4f, 6.2f, 0.0f}, {0.120f, 0.140f, 0.270f, 0.00f}, 7.2f, 1.17f, 2.0f},
-    /* FEW_BF16   */ {{3.5f, 3.6f, 3.5f, 4.9f}, {0.050f, 0.060f, 0.100f, 0.20f}, 5.5f, 0.51f, 0.5f},
-    /* FEW_F32    */ {{3.5f, 3.7f, 3.9f, 5.7f}, {0.080f, 0.104f, 0.190f, 0.50f}, 5.5f, 1.80f, 0.5f},
-    /* FEW_FP8    */ {{3.5f, 3.6f, 3.5f, 5.5f}, {0.036f, 0.050f, 0.088f, 0.20f}, 9.7f, 0.46f, 0.5f},
+    /* FEW_BF16   */ {{3.5f, 3.6f, 3.5f, 5.9f}, {0.050f, 0.060f, 0.100f, 0.25f}, 5.5f, 0.51f, 2.2f},
+    /* FEW_F32    */ {{3.5f, 3.7f, 3.9f, 5.7f}, {0.080f, 0.104f, 0.190f, 0.50f}, 5.5f, 1.80f, 1.1f},
+    /* FEW_FP8    */ {{3.5f, 3.6f, 3.5f, 5.5f}, {0.036f, 0.050f, 0.088f, 0.20f}, 9.7f, 0.46f, 2.4f},
 };
 
 static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {
@@ -433,7 +436,8 @@ static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {
     for (int f = 0; f < (kind == FEW_I16X16 ? 3 : 4); ++f) {
         const float rows = static_cast<float>((g.M + FEW_FORMS[f].tm * 16 - 1) / (FEW_FORMS[f].tm * 16));
         const float cols = static_cast<float>((g.N + FEW_FORMS[f].tn * 16 - 1) / (FEW_FORMS[f].tn * 16));
-        const float per_cu = std::max(1.f, rows * cols * batch / 256.f);
+        float per_cu = std::max(1.f, rows * cols * batch / 256.f);
+        if (f == 3) per_cu = std::ceil(per_cu);  // bound by matrix work and L2: a CU with two workgroups takes as long as two
         const float t = c.start[f] + per_cu * ktiles * c.tile[f] + (per_cu - 1.f) * c.more;
         if (t < *us) {
             *us = t;
@@ -452,7 +456,7 @@ bool few_preferred(const GemmArgs& g, FewKind kind, int batch) {
     const int ktiles = (g.K + 127) / 128;
     float other = (c.other_start + c.other_tile * ktiles) * std::max(1.f, tiles / 256.f);
     // reductions of up to 768 on aligned rows have a kernel of their own with little fixed cost (launch_wreg)
-    if (kind == FEW_I8 && batch == 1 && wreg_applicable(g)) other = 7.3f + static_cast<float>(g.M) * static_cast<float>(g.N) * static_cast<float>(g.K) * 1e-9f;
+    if (kind == FEW_I8 && batch == 1 && wreg_applicable(g)) other = 6.6f + static_cast<float>(g.M) * static_cast<float>(g.N) * static_cast<float>(g.K) * 1.4e-9f;
     float us;
     few_form(g, kind, batch, &us);
     return us < other;
