@@ -351,7 +351,7 @@ class GPUModel:
             q = heads_view(values[grp['q_src']], grp['q_base'])
             k = heads_view(values[grp['k_src']], grp['k_base'])
             v = heads_view(values[grp['v_src']], grp['v_base'])
-            if not _views_are_16_byte_aligned(q, k, v):
+            if not _attention_launch_takes(q, k, v):
                 # slices of slices can start anywhere: the planner sees offsets within the nearest source only
                 self._run_attention_unfused(grp, values, heads_view=(q, k, v))
                 return
@@ -360,7 +360,7 @@ class GPUModel:
             attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode,
                    out=heads_view(out, 0))
             values[grp['out']] = out
-        elif not _views_are_16_byte_aligned(values[tr0['q']], values[tr0['k']], values[tr0['v']]):
+        elif not _attention_launch_takes(values[tr0['q']], values[tr0['k']], values[tr0['v']]):
             self._run_attention_unfused(grp, values)
         else:
             q, k, v = values[tr0['q']], values[tr0['k']], values[tr0['v']]
@@ -369,7 +369,7 @@ class GPUModel:
 
     def _run_attention_unfused(self, grp, values, heads_view=None) -> None:
         """The members of a planned attention group one operator at a time: MatMul, Softmax, MatMul per head, then the
-        concat. Taken when the operands turn out not to be 16-byte aligned views at run time."""
+        concat. Taken when the operands turn out at run time to lie as the fused launch does not take them."""
         execution, graph = self.context.ir.execution, self.context.ir.logical
         for h, tr in enumerate(grp['heads']):
             if heads_view is not None:  # head h of the [batch, heads, seq, d] views, should its slice node come later
@@ -416,16 +416,25 @@ class _Values(dict):
         return view
 
 
-def _views_are_16_byte_aligned(*tensors) -> bool:
-    """What the fused attention launch asks of its operands: 16-byte aligned base addresses and row / head / batch
-    pitches (int8 tensors, so elements are bytes)."""
-    for t in tensors:
+def _attention_launch_takes(q, k, v) -> bool:
+    """Whether the fused attention launches take operands that lie like these; the separate operators take any. Both entry
+    points ask for contiguous int8 rows on 16-byte aligned addresses, row pitches of at least a row, keys (and, for the
+    long one, values) of a head within 2 GiB, and a number of query rows that their grid can count. Shapes, shifts
+    and Softmax parameters are the planner's to check: they are known when the graph is compiled."""
+    rows, keys, dim = int(q.shape[-2]), int(k.shape[-2]), int(q.shape[-1])
+    for t in (q, k, v):
+        stride = t.stride()
+        if stride[-1] != 1 or stride[-2] < dim:
+            return False
         at = t.data_ptr()
-        for st in t.stride()[:-1]:
+        for st in stride[:-1]:
             at |= st  # (a power of two divides all of them if it divides their bitwise or)
         if at % 16:
             return False
-    return True
+    blocks = (rows + 127) // 128
+    for extent in q.shape[:-2]:
+        blocks *= int(extent)
+    return (keys + 32) * max(k.stride(-2), v.stride(-2)) < 1 << 31 and rows <= 1 << 24 and blocks < 1 << 31
 
 
 def _mlp_layers_are_faster(rows: int, layers, on_matrix_units: bool = False) -> bool:

@@ -596,3 +596,117 @@ def test_attention_with_unaligned_head_slices_runs_unfused(oracle):
         # that the slice itself starts 8 bytes into rows of 392 bytes shows at run time, where the executor falls back
         xin = np.clip(np.rint(r.normal(0, 24, (batch, seq, width))), -128, 127).astype(np.int8)
         _graph_check(model, oracle, {'x': xin})
+
+
+def _triple(lead, sq, sk, d):
+    """q, k, v -> MatMul, Softmax (EXP_KQ = 92), MatMul, without a split or a concat around them."""
+    gb = GraphBuilder()
+    q, k, v = (gb.input(n, lead + (s, d), qint(8, 4)) for n, s in (('q', sq), ('k', sk), ('v', sk)))
+    lg = gb.scale(gb.matmul(q, gb.transpose(k, tuple(range(len(lead))) + (len(lead) + 1, len(lead))), qint(8, -3), name='qk'), 1 / 32, qint(8, -3))
+    gb.output(gb.matmul(gb.softmax(lg, qint(8, 8, signed=False), name='sm'), v, qint(8, 4), name='pv'))
+    return gb.build()
+
+
+@pytest.mark.parametrize('seq', [513, 1030])
+@pytest.mark.parametrize('softmax', ['exp', 'hccs'])
+def test_encoder_block_with_a_long_sequence(oracle, seq, softmax):
+    """More tokens than the register-resident attention kernel takes: still one launch for all heads, eager and recorded,
+    and the integers of the graph run operator by operator."""
+    import torch
+
+    model, x = workloads.c5_encoder_block(batch=1, seq=seq, hidden=128, heads=2, ffn=256, softmax=softmax)
+    model.compile()
+    (grp,) = model.context.config['gpu_fusion_plan']['attention']
+    assert len(grp['heads']) == 2 and grp['concat']
+    trace = []
+    dx = {'x': torch.from_numpy(x).cuda()}
+    model.execute(dx, trace=trace)
+    assert [t['kind'] for t in trace].count('attention') == 1 and not any(t['kind'] in ('matmul', 'softmax') for t in trace)
+    got = next(iter(_graph_check(model, oracle, {'x': x}).values()))
+    captured = model.capture(dx)
+    for _ in range(3):
+        replayed = next(iter(captured(dx).values())).cpu().numpy()
+        np.testing.assert_array_equal(replayed.reshape(-1), got.reshape(-1))
+    model.context.config['gpu_fusion_plan'] = {}
+    _graph_check(model, oracle, {'x': x})
+    assert len(np.unique(got)) > 32
+
+
+@pytest.mark.parametrize('lead,sq,sk,d', [((2,), 520, 520, 64), ((1, 3), 5, 1030, 32), ((), 70, 300, 128)])
+def test_long_attention_without_a_concat(oracle, lead, sq, sk, d):
+    """A lone MatMul, Softmax, MatMul triple past the keys of the register-resident kernel; then on operands whose elements
+    or rows lie apart in a way that the launch does not take."""
+    import torch
+
+    r = np.random.default_rng(sk + d)
+    model = _triple(lead, sq, sk, d)
+    x = {n: np.clip(np.rint(r.normal(0, 24, lead + (s, d))), -128, 127).astype(np.int8) for n, s in (('q', sq), ('k', sk), ('v', sk))}
+    want = next(iter(_graph_check(model, oracle, x).values()))
+    dx = {n: torch.from_numpy(a).cuda() for n, a in x.items()}
+    trace = []
+    model.execute(dx, trace=trace)
+    assert [t['kind'] for t in trace] == ['attention']
+    # rows along the last axis in memory, and rows 1 byte off the 16-byte grid between extreme values
+    turned = {n: t.transpose(-1, -2).contiguous().transpose(-1, -2) for n, t in dx.items()}
+    odd = {}
+    for n, t in dx.items():
+        wide = torch.full(tuple(t.shape[:-1]) + (d + 16,), 127, dtype=torch.int8, device='cuda')
+        wide[..., 1:d + 1] = t
+        odd[n] = wide[..., 1:d + 1]
+    for case in (turned, odd, {**dx, 'k': turned['k']}, {**dx, 'v': odd['v']}):
+        got = next(iter(model.execute(case).values())).cpu().numpy()
+        np.testing.assert_array_equal(got.reshape(-1), want.reshape(-1))
+
+
+def test_long_attention_whose_keys_span_more_than_the_launch_takes():
+    """32768 keys in rows of 64 KiB: a head's keys span 2 GiB, which the fused launch refuses; the graph runs operator by
+    operator and gives what the fused launch gives on a compact copy of the same keys and values."""
+    import torch
+
+    from aie4ml_amd import ops
+
+    sk, d = 32768, 64
+    model = _triple((1,), 8, sk, d)
+    model.compile()
+    (grp,) = model.context.config['gpu_fusion_plan']['attention']
+    gen = torch.Generator(device='cuda').manual_seed(5)
+    q, k, v = ((torch.randn((1, rows, d), generator=gen, device='cuda') * 24).round().clamp(-128, 127) for rows in (8, sk, sk))
+    k[:, 7::4096] = (q * 5).clamp(-128, 127)  # one key per query stands out: 32768 equal probabilities would all round to zero
+    q, k, v = (t.to(torch.int8) for t in (q, k, v))
+    wide = torch.empty((1, sk, 1 << 16), dtype=torch.int8, device='cuda')
+    wide[..., 64:128], wide[..., 256:320] = k, v
+    got = next(iter(model.execute({'q': q, 'k': wide[..., 64:128], 'v': wide[..., 256:320]}).values()))
+    want = next(iter(model.execute({'q': q, 'k': k, 'v': v}).values()))
+    assert torch.equal(got, want) and len(torch.unique(want)) > 32
+    with pytest.raises(NotImplementedError, match='2 GiB'):
+        ops.attention_long(q, wide[..., 64:128], v, 6, 'floor', {'kind': 'exp', 'exp_kq': 23}, 7, 'floor')
+
+
+@pytest.mark.parametrize('seq', [64, 520])
+@pytest.mark.parametrize('case', ['unaligned', 'slice_is_output', 'slice_has_a_reader'])
+def test_head_slices_made_on_demand(oracle, case, seq):
+    """Heads that run as one launch are read from their common source and their slices are not made, unless the launch does
+    not take them (slices that start 8 bytes into a row), a slice is itself a graph output, or another operator reads it."""
+    r = np.random.default_rng(seq + len(case))
+    batch, heads, d = 2, 2, 64
+    pad = 8 if case == 'unaligned' else 16
+    gb = GraphBuilder()
+    x = gb.input('x', (batch, seq, pad + 3 * heads * d), qint(8, 4))
+    _pad, q, k, v = gb.split(x, -1, [pad, heads * d, heads * d, heads * d], name='qkv_split')
+    qs, ks, vs = (gb.split(t, -1, [d] * heads, name=f'{n}_heads') for t, n in ((q, 'q'), (k, 'k'), (v, 'v')))
+    outs = []
+    for h in range(heads):
+        lg = gb.matmul(qs[h], gb.transpose(ks[h], (0, 2, 1), name=f'kt{h}'), qint(8, -3), name=f'qk{h}')
+        pr = gb.softmax(gb.scale(lg, 1 / 32, name=f'temp{h}'), qint(8, 8, signed=False), name=f'sm{h}')
+        outs.append(gb.matmul(pr, vs[h], qint(8, 4), name=f'pv{h}'))
+    gb.output(gb.concat(outs, -1, name='cat'))
+    if case == 'slice_is_output':
+        gb.output(vs[1])
+    elif case == 'slice_has_a_reader':
+        gb.output(gb.add(qs[0], vs[1], qint(8, 4), name='extra'))
+    model = gb.build()
+    model.compile()
+    (grp,) = model.context.config['gpu_fusion_plan']['attention']
+    assert grp['concat'] and len(grp['heads']) == heads
+    xin = np.clip(np.rint(r.normal(0, 24, (batch, seq, pad + 3 * heads * d))), -128, 127).astype(np.int8)
+    _graph_check(model, oracle, {'x': xin})

@@ -436,6 +436,29 @@ def test_attention_plan_merges_heads():
     assert ctx.config['gpu_fusion_plan']['attention'] == []
 
 
+def test_attention_launch_takes_what_the_entry_points_take():
+    """Operands that the fused attention entry points refuse at their launch go to the separate operators: rows off the
+    16-byte grid, elements apart, rows that overlap, keys or values of a head that span 2 GiB, too many blocks of rows."""
+    import torch
+
+    from aie4ml_amd.model import _attention_launch_takes
+
+    def operand(rows, row_pitch=64, lead=(1, 2), element=1):  # strides and shapes only, no memory behind them
+        strides = tuple(rows * row_pitch for _ in lead) + (row_pitch, element)
+        return torch.empty_strided(lead + (rows, 64), strides, dtype=torch.int8, device='meta')
+
+    q, k = operand(128), operand(32768)
+    assert _attention_launch_takes(q, k, k) and _attention_launch_takes(operand(1), operand(1), operand(1))
+    assert _attention_launch_takes(operand(1 << 24), k, k)
+    widest = (1 << 31) // (32768 + 32) // 16 * 16  # 65472: 32800 rows of it are less than 2 GiB
+    assert _attention_launch_takes(q, operand(32768, widest), operand(32768, widest))
+    for bad in (operand(32768, widest + 16), operand(32768, 65536), operand(32768, 72), operand(32768, 48), operand(32768, 64, element=2)):
+        assert not _attention_launch_takes(q, bad, k), bad.stride()
+        assert not _attention_launch_takes(q, k, bad), bad.stride()
+    assert not _attention_launch_takes(operand((1 << 24) + 1), k, k)
+    assert not _attention_launch_takes(operand(128, lead=(65536, 32768)), operand(16, lead=(65536, 32768)), operand(16, lead=(65536, 32768)))
+
+
 class GraphHolder:
     """Adapts a model to the `gb.ctx` attribute lower() expects."""
 
