@@ -44,7 +44,7 @@ struct Gemm16Args {
     // batched use (dynamic MatMul): element strides between consecutive problems, blockIdx.y = problem
     int64_t stride_a, stride_w, stride_colsum, stride_y;
     int shift;  // used when `shifts` is null (MatMul: one host-side shift)
-    int trans_a;   // RAGGED kernels: A is stored transposed, [K][lda]
+    int trans_a;   // A is stored transposed, [K][lda]
 };
 
 // 128 x BN output tile, K step 64, 4 waves (2 x 2) of 64 x BN / 2, double-buffered LDS holding the two byte
@@ -58,14 +58,16 @@ __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
 }
 
 // ROWS: how A is read. 0: rows 16-byte aligned, K a multiple of 16. 1: any address, any K of 8 or more (one unaligned load
-// per chunk, the chunk that crosses a row's end moved into place as it is staged). 2: stored transposed, shorter, or a pitch
-// beyond 32-bit offsets (loads in branches). The packed weights are aligned and zero padded to 16 in every form.
+// per chunk, the chunk that crosses a row's end moved into place as it is staged). 2: rows shorter than that or a pitch beyond
+// 32-bit offsets (loads in branches). 3: stored transposed (gathered element by element). The packed weights are aligned and zero
+// padded to 16 in every form. (2 and 3 chosen between at run time inside one instance spilled registers: 8192 x 1024 -> 1000
+// transposed 118 us, 94 us as a form of its own.)
 // A K tile is 0.2 us of matrix work and a load takes 1 us and more, so forms 0 and 1 have two K tiles on their way in
 // registers beside the one in LDS, fetched through buffer descriptors (past K or past the last row reads as zero: no load
 // stands in a branch, so every wait counts exactly). Rate by size in the comment at the launch.
 template <int ROWS, int BN>
 __global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm16Args g) {
-    constexpr bool RAGGED = ROWS == 2;
+    constexpr bool RAGGED = ROWS >= 2;
     constexpr int SETS = RAGGED ? 1 : 2;
     constexpr int BM = 128, BK = 64, PITCH = BK + 16, TN = BN / 64, LB = BN / 64;  // a wave: 64 rows, BN / 2 columns
     select_problem(g, blockIdx.y);
@@ -131,9 +133,8 @@ __global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm1
         for (int i = 0; i < 4; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
             const int gm = min(m0 + row, g.M - 1);
-            ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
-                              : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                  (g.K - (k0 + kc)) * 2, g.K * 2);
+            if constexpr (ROWS == 3) ra[i] = load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2);
+            else ra[i] = load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc), (g.K - (k0 + kc)) * 2, g.K * 2);
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm1
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
-            if (ROWS != 0 && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
+            if ((ROWS == 1 || ROWS == 2) && k0 + BK > g.K) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             // eight int16 in four dwords -> their eight high bytes and eight low bytes
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             v2i hi = {static_cast<int>(__builtin_amdgcn_perm(w1, w0, 0x07050301u)), static_cast<int>(__builtin_amdgcn_perm(w3, w2, 0x07050301u))};
@@ -215,7 +216,11 @@ __global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm1
             load_tile(set, (kt + 1 + SETS) * BK);
         }
         half(st, 1);
-        if (RAGGED && more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+        if (RAGGED) {
+            if (more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+            __syncthreads();
+            return;
+        }
         __builtin_amdgcn_sched_barrier(0);
         wait_lgkmcnt0();  // (a __syncthreads may also wait for the loads)
         __builtin_amdgcn_s_barrier();
@@ -259,6 +264,7 @@ static void launch_tiled_i16i8(const Gemm16Args& g, unsigned batch, bool aligned
     const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23);
     if (near && aligned) launch_i16i8_form<0, 64>(g, batch, stream);
     else if (near && !g.trans_a && g.K >= 8) launch_i16i8_form<1, 64>(g, batch, stream);
+    else if (g.trans_a) launch_i16i8_form<3, 128>(g, batch, stream);
     else launch_i16i8_form<2, 128>(g, batch, stream);
 }
 
@@ -302,7 +308,7 @@ struct Gemm16x16Args {
     int shift_stride, relu, out_kind, mode;
     int64_t stride_a, stride_w, stride_colsum, stride_y;  // batched use, as above
     int shift;                                            // used when `shifts` is null
-    int trans_a;                                          // RAGGED kernels: A is stored transposed, [K][lda]
+    int trans_a;                                          // A is stored transposed, [K][lda]
 };
 
 __device__ __forceinline__ long long round_shift64(long long v, int s, int mode) {
@@ -478,7 +484,7 @@ __device__ __forceinline__ void select_problem(Gemm16x16Args& g, int b) {
 // ROWS and the two K tiles on their way in registers: as in gemm_i16i8_kernel.
 template <int ROWS>
 __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
-    constexpr bool RAGGED = ROWS == 2;
+    constexpr bool RAGGED = ROWS >= 2;
     constexpr int SETS = RAGGED ? 1 : 2;
     constexpr int BM = 64, BN = 128, BK = 64, PITCH = BK + 16;
     select_problem(g, blockIdx.y);
@@ -544,9 +550,8 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
         for (int i = 0; i < 2; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
             const int gm = min(m0 + row, g.M - 1);
-            ra[i] = g.trans_a ? load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2)
-                              : load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc),
-                                                  (g.K - (k0 + kc)) * 2, g.K * 2);
+            if constexpr (ROWS == 3) ra[i] = load_chunk_transposed(reinterpret_cast<const int8_t*>(g.A + gm), g.lda * 2, k0 + kc, g.K, 2);
+            else ra[i] = load_chunk_ragged(reinterpret_cast<const int8_t*>(g.A + static_cast<int64_t>(gm) * g.lda + k0 + kc), (g.K - (k0 + kc)) * 2, g.K * 2);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -566,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int c = tid + i * 256, row = c >> 3, kc = (c & 7) * 8;
-            if (ROWS != 0 && k0 + BK > g.K && !g.trans_a) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
+            if ((ROWS == 1 || ROWS == 2) && k0 + BK > g.K) ra[i] = chunk_in_place(ra[i], (g.K - (k0 + kc)) * 2, g.K * 2);
             const unsigned w0 = ra[i][0], w1 = ra[i][1], w2 = ra[i][2], w3 = ra[i][3];
             // beyond K both planes are zero, so the row sums stay exact: the low bytes are biased where k < K only
             const int live = min(max(g.K - (k0 + kc), 0), 8);  // elements of this chunk below K (0 or 8 where K is in whole chunks)
@@ -635,7 +640,11 @@ __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {
             load_tile(set, (kt + 1 + SETS) * BK);
         }
         half(st, 1);
-        if (RAGGED && more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+        if (RAGGED) {
+            if (more) store_tile(0, (kt + 1) & 1, (kt + 1) * BK);
+            __syncthreads();
+            return;
+        }
         __builtin_amdgcn_sched_barrier(0);
         wait_lgkmcnt0();
         __builtin_amdgcn_s_barrier();
@@ -704,6 +713,7 @@ static void launch_tiled_i16i16(const Gemm16x16Args& g, dim3 grid, bool aligned,
     const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23);
     if (near && aligned) gemm_i16i16_kernel<0><<<grid, 256, lds, stream>>>(g);
     else if (near && !g.trans_a && g.K >= 8) gemm_i16i16_kernel<1><<<grid, 256, lds, stream>>>(g);
+    else if (g.trans_a) gemm_i16i16_kernel<3><<<grid, 256, lds, stream>>>(g);
     else gemm_i16i16_kernel<2><<<grid, 256, lds, stream>>>(g);
 }
 
