@@ -10,8 +10,8 @@
 //
 // Large problems with whole 128-element K tiles run on the software-pipelined kernel of gemm_rs.hpp with the
 // planes as rows (and, for int16 weights, columns) of its tile: I16Policy beside the int8 policy whose epilogue
-// it shares, I16x16Policy below. The kernels in this file take every other shape: K a multiple of 16 the
-// double-buffered tiled ones, anything else one thread per output.
+// it shares, I16x16Policy below; small outputs go to gemm_few.hip. The tiled kernels in this file take every other shape; weights that were
+// not packed by this library (rows off the 16-byte grid) are left to one thread per output.
 #include <cstdlib>
 #include <algorithm>
 #include "common.hpp"
@@ -47,8 +47,6 @@ struct Gemm16Args {
     int trans_a;   // A is stored transposed, [K][lda]
 };
 
-// 128 x BN output tile, K step 64, 4 waves (2 x 2) of 64 x BN / 2, double-buffered LDS holding the two byte
-// planes of A and the weight tile.
 __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
     const int obytes = (g.out_kind == A4G_I16 || g.out_kind == A4G_U16) ? 2 : 1;
     g.A += b * g.stride_a;
@@ -57,6 +55,8 @@ __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
     g.Y = static_cast<int8_t*>(g.Y) + b * g.stride_y * obytes;
 }
 
+// 128 x BN output tile, K step 64, 4 waves (2 x 2) of 64 x BN / 2, double-buffered LDS holding the two byte planes of A and
+// the weight tile.
 // ROWS: how A is read. 0: rows 16-byte aligned, K a multiple of 16. 1: any address, any K of 8 or more (one unaligned load
 // per chunk, the chunk that crosses a row's end moved into place as it is staged). 2: rows shorter than that or a pitch beyond
 // 32-bit offsets (loads in branches). 3: stored transposed (gathered element by element). The packed weights are aligned and zero
@@ -64,7 +64,7 @@ __device__ __forceinline__ void select_problem(Gemm16Args& g, int b) {
 // transposed 118 us, 94 us as a form of its own.)
 // A K tile is 0.2 us of matrix work and a load takes 1 us and more, so forms 0 and 1 have two K tiles on their way in
 // registers beside the one in LDS, fetched through buffer descriptors (past K or past the last row reads as zero: no load
-// stands in a branch, so every wait counts exactly). Rate by size in the comment at the launch.
+// stands in a branch, so every wait counts exactly). BN: 64 or 128 columns, chosen by wide_tiles_i16i8, where the times are.
 template <int ROWS, int BN>
 __global__ __launch_bounds__(256, BN == 64 ? 3 : 2) void gemm_i16i8_kernel(Gemm16Args g) {
     constexpr bool RAGGED = ROWS >= 2;
@@ -258,12 +258,22 @@ static void launch_i16i8_form(const Gemm16Args& g, unsigned batch, hipStream_t s
     gemm_i16i8_kernel<ROWS, BN><<<grid, 256, tiled16_lds_bytes(g.K, 256 + BN, 128, BN), stream>>>(g);
 }
 
+// Tiles of 128 x 128 read less and multiply more per load, tiles of 128 x 64 make twice as many workgroups of which three instead of two
+// share a CU. A CU's time goes with the workgroups it gets; one of 128 columns costs what 1.3 (long reductions) to 1.9 (short ones)
+// of 64 cost. Measured (64 / 128 columns, us): 512 x 768 -> 2048 10.2 / 13.0, 2048 x 768 -> 3072 19.8 / 20.5, 2048 x 2000 -> 3072
+// 44.7 / 39.3, 8192 x 768 -> 768 24.5 / 21.9, 8192 x 2000 -> 3072 157.6 / 122.6, 16384 x 60 -> 2048 33.9 / 33.0.
+static bool wide_tiles_i16i8(int64_t M, int64_t N, int64_t K, unsigned batch) {
+    const int64_t rows = (M + 127) / 128 * batch;
+    const int64_t wide = (rows * ((N + 127) / 128) + 255) / 256, narrow = (rows * ((N + 63) / 64) + 255) / 256;  // workgroups of a CU
+    return static_cast<float>(wide) < std::min(0.525f + 0.000143f * static_cast<float>(K), 0.8f) * static_cast<float>(narrow);
+}
+
 // `aligned`: A stored row by row, rows 16-byte aligned, K a multiple of 16. The forms that fetch through descriptors hold a
 // tile's 128 rows within 30-bit offsets.
 static void launch_tiled_i16i8(const Gemm16Args& g, unsigned batch, bool aligned, hipStream_t stream) {
-    const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23);
-    if (near && aligned) launch_i16i8_form<0, 64>(g, batch, stream);
-    else if (near && !g.trans_a && g.K >= 8) launch_i16i8_form<1, 64>(g, batch, stream);
+    const bool near = g.lda <= (1 << 22) && g.ldwt <= (1 << 23), wide = wide_tiles_i16i8(g.M, g.N, g.K, batch);
+    if (near && aligned) wide ? launch_i16i8_form<0, 128>(g, batch, stream) : launch_i16i8_form<0, 64>(g, batch, stream);
+    else if (near && !g.trans_a && g.K >= 8) wide ? launch_i16i8_form<1, 128>(g, batch, stream) : launch_i16i8_form<1, 64>(g, batch, stream);
     else if (g.trans_a) launch_i16i8_form<3, 128>(g, batch, stream);
     else launch_i16i8_form<2, 128>(g, batch, stream);
 }
@@ -470,8 +480,6 @@ static bool rs_i16i16_applicable(const GemmArgs& g, int batch) {
            static_cast<int64_t>((g.M + 127) / 128) * ((g.N + 127) / 128) * batch >= 192;
 }
 
-// 64 x 128 output tile, K step 64, 4 waves (2 x 2) of 32 x 64, double-buffered LDS with the two byte planes
-// of both operands. Requires K % 16 == 0, 16-byte aligned rows.
 __device__ __forceinline__ void select_problem(Gemm16x16Args& g, int b) {
     const int obytes = (g.out_kind == A4G_I16 || g.out_kind == A4G_U16) ? 2 : 1;
     g.A += b * g.stride_a;
@@ -481,6 +489,7 @@ __device__ __forceinline__ void select_problem(Gemm16x16Args& g, int b) {
     g.Y = static_cast<int8_t*>(g.Y) + b * g.stride_y * obytes;
 }
 
+// 64 x 128 output tile, K step 64, 4 waves (2 x 2) of 32 x 64, double-buffered LDS with the two byte planes of both operands.
 // ROWS and the two K tiles on their way in registers: as in gemm_i16i8_kernel.
 template <int ROWS>
 __global__ __launch_bounds__(256, 2) void gemm_i16i16_kernel(Gemm16x16Args g) {

@@ -1444,3 +1444,25 @@ def test_dense_with_two_k_tiles_ahead(ops, oracle, kind, K):
     want = oracle.dense(np.ascontiguousarray(A), W, None, np.array([shift]), 'conv_even', out=out)
     for x in (dev(np.ascontiguousarray(A)), dev(wide)[:, 1:K + 1]):
         assert np.array_equal(host(ops.dense(x, p, 'conv_even', out_kind=out)), want), tuple(x.stride())
+
+
+@pytest.mark.parametrize('M,N,batch', [(3000, 330, 1), (8200, 330, 1), (1000, 200, 3), (2000, 330, 8)])
+@pytest.mark.parametrize('K', [8, 64, 129, 520])
+def test_int16_tiles_of_both_widths(ops, oracle, M, N, batch, K):
+    """int16 x int8 with more outputs than the kernel for small ones takes, on tiles of 64 columns (the first and third size) and of 128 (the
+    others): rows and columns off the tiles, K below one K tile, on and off the 16-byte grid, rows aligned and at odd
+    elements between extreme values; Dense and, with several problems, MatMul."""
+    r = rng(M + N + K)
+    info = np.iinfo(np.int16)
+    W = gauss8(r, 40, (batch, K, N))
+    wide = np.where(np.arange(K + 16) % 2, info.max, info.min).astype(np.int16)[None].repeat(batch * M, 0)
+    A = wide[:, 1:K + 1] = r.integers(info.min, info.max + 1, (batch * M, K)).astype(np.int16)
+    A = np.ascontiguousarray(A)
+    if batch > 1:
+        got = host(ops.matmul(dev(A.reshape(batch, M, K)), dev(W), 16, 'conv_even', out_kind='int16'))
+        assert np.array_equal(got, oracle.matmul(A.reshape(batch, M, K), W, 16, 'conv_even', out='int16'))
+        return
+    p = ops.pack_dense(dev(W[0]), None, 16)
+    want = oracle.dense(A, W[0], None, np.array([16]), 'conv_even', out='int16')
+    for x in (dev(A), dev(wide)[:, 1:K + 1]):
+        assert np.array_equal(host(ops.dense(x, p, 'conv_even', out_kind='int16')), want), tuple(x.stride())
