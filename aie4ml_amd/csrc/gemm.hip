@@ -817,8 +817,10 @@ static hipError_t launch_rs_u(const GemmArgs& g, int batch, hipStream_t stream) 
 }
 
 bool rs_i16i8_applicable(const GemmArgs& g, int batch) {
-    // whole 128-element K tiles, 16-byte aligned rows, and enough 128 x 256 tiles to give every CU one; from K = 1024 on
-    // (measured 3-7 % ahead of the tiled kernel there, level or behind for shorter reductions and for narrow outputs)
+    // whole 128-element K tiles, 16-byte aligned rows, and enough 128 x 256 tiles to give every CU one; from K = 1024 on. Against the
+    // tiled kernel there (pipelined / tiled, us): 8192 x 1024 -> 1024 22.8 / 25.4, 2048 x 4096 -> 3072 53.9 / 68.7, 16384 x 2048 -> 1024
+    // 71.5 / 79.1; behind where its larger tiles leave most of a round empty (4096 x 1024 -> 3072 37.5 / 35.9). At K = 768 both
+    // occur (8192 -> 768 17.6 / 19.4, 16384 -> 768 32.0 / 30.0), below it the tiled one is ahead or level
     return g.K % 128 == 0 && g.K >= 1024 && g.N >= 192 && g.lda % 16 == 0 && g.stride_a % 16 == 0 && g.ldb % 16 == 0 &&
            g.stride_b % 16 == 0 && aligned16(g.A) && aligned16(g.Bt) && g.colsum != nullptr &&
            static_cast<int64_t>((g.M + 127) / 128) * ((g.N + 255) / 256) * batch >= 192;
@@ -839,6 +841,11 @@ static hipError_t launch_dtl(const GemmArgs& g, int batch, hipStream_t stream) {
     return g.a_unsigned ? launch_dtl_u<BM, BN, BK, WAVES_M, WAVES_N, STAGES, true>(g, batch, stream)
                         : launch_dtl_u<BM, BN, BK, WAVES_M, WAVES_N, STAGES, false>(g, batch, stream);
 }
+
+// The pipelined kernel takes every K of at least a chunk: 8192 x 17 -> 777 12.4 us, 25.9 on the older tiled one; 8192 x 255 -> 2048
+// 25.6 and 38.3. Only short reductions of hundreds of small problems, where its registers let fewer of them share a CU, stay on
+// that (768 x 100 x 32 x 100: 16.6 us, 17.9 pipelined).
+static bool tiled_is_ahead(const GemmArgs& g, int batch) { return g.K < 16 || (g.K < 160 && batch >= 512); }
 
 // Picks a kernel and tile shape for the problem. variant: 0 = automatic; 1..4 force a tile shape (tuning only,
 // through the A4G_GEMM_VARIANT environment variable; a forced shape whose kernel's K granularity does not
@@ -872,11 +879,10 @@ static hipError_t launch_gemm_nt(const GemmArgs& g, int batch, hipStream_t strea
     case 2:  // 128 x 128
         if (k128) return launch_rs<128, 128, 2, 2>(g, batch, stream);
         if (k64) return launch_dtl<128, 128, 64, 2, 2, 4>(g, batch, stream);
-        if (g.K >= 256) {  // K in whole 16-byte chunks but not whole tiles: as above
-            return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, true>(g, batch, stream)
-                                : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, true>(g, batch, stream);
-        }
-        return launch_tiled<128, 128, 64, 2, 2>(g, batch, stream);
+        if (tiled_is_ahead(g, batch)) return launch_tiled<128, 128, 64, 2, 2>(g, batch, stream);
+        // K in whole 16-byte chunks but not whole tiles: as above
+        return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, true>(g, batch, stream)
+                            : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, true>(g, batch, stream);
     case 4:  // 128 x 192
         if (k128) return g.a_unsigned ? launch_rs_u<128, 192, 2, 2, true, true>(g, batch, stream)
                                       : launch_rs_u<128, 192, 2, 2, false, true>(g, batch, stream);
@@ -906,8 +912,7 @@ static int env_variant() {
 
 // K off the 16-byte grid or rows at any address: same tiles, chunk loads at any address.
 static hipError_t launch_ragged(const GemmArgs& g, int batch, hipStream_t stream) {
-    // from two K tiles on the pipelined kernel is ahead (25 us against 31 us at 8192 x 1024 x 1008)
-    if (g.K < 256) return launch_tiled<128, 128, 64, 2, 2, true>(g, batch, stream);
+    if (tiled_is_ahead(g, batch)) return launch_tiled<128, 128, 64, 2, 2, true>(g, batch, stream);
     if (whole_chunk_rows(g.Bt, g.ldb, g.stride_b, g.K))
         return g.a_unsigned ? launch_rs_policy<I8Policy<true>, 128, 128, 2, 2, false, false, 2>(g, batch, stream)
                             : launch_rs_policy<I8Policy<false>, 128, 128, 2, 2, false, false, 2>(g, batch, stream);

@@ -473,8 +473,8 @@ struct I16x16Policy {
 };
 
 static bool rs_i16i16_applicable(const GemmArgs& g, int batch) {
-    // the pipelined kernel pays from K = 1024 on (3-10 % ahead of the tiled one; a few per cent behind at K <= 512),
-    // and only when the tile's 128 columns are mostly used (N = 64: 299 us against 229 us)
+    // the pipelined kernel pays from K = 1024 on (pipelined / tiled, us: 4096 x 1024 -> 768 20.1 / 23.7, 8192 x 4096 -> 3072 380 / 468, 2048 x
+    // 1024 -> 3072 38.4 / 38.2; at K = 512 8192 -> 768 26.8 / 25.1), and only when the tile's 128 columns are mostly used
     return g.K % 128 == 0 && g.K >= 1024 && g.N >= 192 && g.K <= 32768 && g.lda % 16 == 0 && g.stride_a % 16 == 0 && g.ldb % 16 == 0 &&
            g.stride_b % 16 == 0 && aligned16(g.A) && aligned16(g.Bt) && aligned16(g.Bt_lo) &&
            static_cast<int64_t>((g.M + 127) / 128) * ((g.N + 127) / 128) * batch >= 192;

@@ -1466,3 +1466,28 @@ def test_int16_tiles_of_both_widths(ops, oracle, M, N, batch, K):
     want = oracle.dense(A, W[0], None, np.array([16]), 'conv_even', out='int16')
     for x in (dev(A), dev(wide)[:, 1:K + 1]):
         assert np.array_equal(host(ops.dense(x, p, 'conv_even', out_kind='int16')), want), tuple(x.stride())
+
+
+@pytest.mark.parametrize('K', [15, 16, 17, 48, 79, 112, 130, 208, 255])
+@pytest.mark.parametrize('kind', ['int8', 'uint8'])
+def test_short_reductions_on_many_tiles(ops, oracle, kind, K):
+    """Reductions of one to two K tiles with more outputs than the kernel for small ones takes: Dense with two-byte results (so that no
+    other kernel does), rows on and off the 16-byte grid between extreme values, and MatMul on two and on hundreds of problems."""
+    r = rng(K + len(kind))
+    adt = {'int8': np.int8, 'uint8': np.uint8}[kind]
+    info = np.iinfo(adt)
+    M, N = 4100, 520
+    W = gauss8(r, 40, (K, N))
+    p = ops.pack_dense(dev(W), dev(r.integers(-2**12, 2**12, N).astype(np.int32)), 6)
+    bias = host(p.bias)
+    wide = np.where(np.arange(K + 16) % 2, info.max, info.min).astype(adt)[None].repeat(M, 0)
+    A = wide[:, 1:K + 1] = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+    A = np.ascontiguousarray(A)
+    want = oracle.dense(A, W, bias, np.array([6]), 'conv_even', out='int16')
+    for x in (dev(A), dev(wide)[:, 1:K + 1]):
+        assert np.array_equal(host(ops.dense(x, p, 'conv_even', out_kind='int16')), want), tuple(x.stride())
+    for batch, M, N in ((2, 1030, 300), (600, 33, 20)):
+        A = r.integers(info.min, info.max + 1, (batch, M, K)).astype(adt)
+        B = gauss8(r, 40, (batch, N, K))
+        got = host(ops.matmul(dev(A), dev(B), 6, 'conv_even', trans_b=True, out_kind='int16'))
+        assert np.array_equal(got, oracle.matmul(A, B, 6, 'conv_even', trans_b=True, out='int16')), batch
