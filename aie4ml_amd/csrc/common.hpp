@@ -314,14 +314,26 @@ __device__ __forceinline__ v4i drop_front_bytes(v4i r, int s) {
 // One 16-byte chunk of an operand row of `row` bytes whose length is not a multiple of 16 or whose start is not aligned:
 // `rem` bytes of the row are left at p. A chunk that crosses the end of the row is fetched as the row's last 16 bytes
 // (no byte outside the row is touched, no branch around the load) and moved into place by chunk_in_place, which the
-// caller applies where it first uses the chunk. Rows shorter than 16 bytes are read byte by byte.
+// caller applies where it first uses the chunk. A row of less than 16 bytes is its first and its last piece of 8, 4 or 2 bytes, which
+// overlap (600 problems of 130 x 8 x 200: 70.8 us byte by byte, 58.8 us this way).
 __device__ __forceinline__ v4i load_chunk_ragged(const int8_t* p, int rem, int row) {
     if (row >= 16) return load16_any(p + min(rem - 16, 0));
-    v4i r = {0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < 15; ++b)
-        if (b < rem) r[b >> 2] |= static_cast<int>(static_cast<unsigned>(static_cast<uint8_t>(p[b])) << (8 * (b & 3)));
-    return r;
+    typedef unsigned long long u64_any __attribute__((aligned(1)));
+    typedef unsigned u32_any __attribute__((aligned(1)));
+    typedef unsigned short u16_any __attribute__((aligned(1)));
+    if (rem <= 0) return v4i{0, 0, 0, 0};  // (the only chunk of a short row starts at its first byte)
+    unsigned long long lo, hi = 0;
+    if (row >= 8) {
+        lo = *reinterpret_cast<const u64_any*>(p);
+        hi = (*reinterpret_cast<const u64_any*>(p + row - 8) >> 1) >> (8 * (16 - row) - 1);  // its last row - 8 bytes
+    } else if (row >= 4) {
+        lo = *reinterpret_cast<const u32_any*>(p) |
+             static_cast<unsigned long long>(*reinterpret_cast<const u32_any*>(p + row - 4)) >> (8 * (8 - row)) << 32;
+    } else {
+        lo = static_cast<uint8_t>(p[0]);
+        if (row >= 2) lo = *reinterpret_cast<const u16_any*>(p) | static_cast<unsigned>(static_cast<uint8_t>(p[row - 1])) << (8 * (row - 1));
+    }
+    return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
 }
 __device__ __forceinline__ v4i chunk_in_place(const v4i& r, int rem, int row) {
     return row >= 16 && rem < 16 ? drop_front_bytes(r, 16 - rem) : r;

@@ -1491,3 +1491,24 @@ def test_short_reductions_on_many_tiles(ops, oracle, kind, K):
         B = gauss8(r, 40, (batch, N, K))
         got = host(ops.matmul(dev(A), dev(B), 6, 'conv_even', trans_b=True, out_kind='int16'))
         assert np.array_equal(got, oracle.matmul(A, B, 6, 'conv_even', trans_b=True, out='int16')), batch
+
+
+@pytest.mark.parametrize('K', range(1, 16))
+def test_rows_shorter_than_a_chunk(ops, oracle, K):
+    """Operand rows of 1 to 15 bytes (int16 ones up to 30), which are fetched in overlapping pieces: MatMul on many small problems, Dense
+    windows at odd addresses between extreme values, and Softmax."""
+    r = rng(1000 + K)
+    for adt, bdt in ((np.int8, np.int8), (np.uint8, np.int8), (np.int16, np.int8), (np.int16, np.int16)):
+        info = np.iinfo(adt)
+        A = r.integers(info.min, info.max + 1, (520, 33, K)).astype(adt)
+        B = (r.integers(-32768, 32768, (520, 20, K)).astype(np.int16) if bdt == np.int16 else gauss8(r, 40, (520, 20, K)))
+        shift = 14 if bdt == np.int16 else 10 if adt == np.int16 else 4
+        got = host(ops.matmul(dev(A), dev(B), shift, 'conv_even', trans_b=True, out_kind='int16'))
+        assert np.array_equal(got, oracle.matmul(A, B, shift, 'conv_even', trans_b=True, out='int16')), (adt, bdt)
+        wide = np.where(np.arange(K + 2) % 2, info.max, info.min).astype(adt)[None].repeat(9000, 0)
+        X = wide[:, 1:K + 1] = r.integers(info.min, info.max + 1, (9000, K)).astype(adt)
+        W = np.ascontiguousarray(B[:13].reshape(-1, K)[:260].T)
+        got = host(ops.dense(dev(wide)[:, 1:K + 1], ops.pack_dense(dev(W), None, shift), 'conv_even', out_kind='int16'))
+        assert np.array_equal(got, oracle.dense(np.ascontiguousarray(X), W, None, np.array([shift]), 'conv_even', out='int16')), (adt, bdt)
+    x = gauss8(r, 40, (1000, K))
+    assert np.array_equal(host(ops.softmax_exp(dev(x), 23)), oracle.softmax_exp(x, 23))
