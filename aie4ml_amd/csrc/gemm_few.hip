@@ -431,8 +431,7 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
             switch (form) {
             case 0: return launch_few_tile<KIND, 4, 1, 1, 4, true>(g, batch, stream);
             case 1: return launch_few_tile<KIND, 4, 2, 1, 3, true>(g, batch, stream);
-            case 2: return launch_few_tile<KIND, 4, 2, 2, 2, true>(g, batch, stream);
-            default: return launch_few_tile<KIND, 4, 4, 4, 1, true>(g, batch, stream);
+            default: return launch_few_tile<KIND, 4, 2, 2, 2, true>(g, batch, stream);
             }
         }
     }
@@ -446,40 +445,54 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
     }
 }
 
-// Fitted to measurements (38 shapes of 1 to 8192 rows, 48 to 5000 inputs, 10 to 4096 outputs in every format, and a grid of 17 to 4096
-// rows, 32 to 2048 inputs, 64 to 2048 outputs: 1716 shapes in int8, 140 in each floating-point format): a launch of form f
-// takes start[f] us, plus tile[f] us for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus `more` us
-// for every workgroup of a CU after its first; the tiled kernels take other_start us plus other_tile us for every K
-// tile, times the share of the chip that their 128 x 128 tiles need if that is more than all of it.
-// Measured, this kernel / the tiled ones, us: 16 x 4096 -> 4096 int8 5.4 / 22.3, int16 7.5 / 51, bfloat16 6.7 / 38, float32
-// 14 / 235, fp8 4.6 / 24; 128 x 3072 -> 768 int8 5.7 / 18.7; 128 x 768 -> 768 int8 4.6 / 7.7; 1024 x 768 -> 768 int8 6.9 / 7.8;
-// 2048 x 768 -> 768 int8 10.1 / 9.6 (not taken); 512 x 4096 -> 4096 int8 21.5 / 26.4; 100 x 5000 -> 10 int8 5.7 / 34;
-// 2048 x 256 -> 768 int8 9.4 / 7.3, 4096 x 64 -> 1536 bfloat16 21.0 / 9.0, 4096 x 256 -> 1536 fp8 20.7 / 13.4 (none of them taken).
+// What a launch takes, in us: `start`, plus `tile` for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus
+// `more` for every workgroup of a CU after its first. The tiled kernels by the same law with their 128 x 128 tiles. Fitted to 800 random
+// sizes in every format (2400 in int8) at which every form and the tiled kernel were timed: 1 to 16384 rows, 32 to 8192 inputs, 8 to
+// 8192 outputs, from a workgroup in all to hundreds for a CU; where the law is coarse the constants are the ones that pick best.
+// What is picked is within 0.1 % of the fastest on average (int8 and int16 0.2 %, float32 0.7 %). Measured, this kernel / the tiled ones, us:
+// 16 x 4096 -> 4096 int8 5.4 / 22.3, int16 7.5 / 51, bfloat16 6.7 / 38, float32 14 / 235, fp8 4.6 / 24; 128 x 768 -> 768 int8
+// 4.6 / 7.7; 1024 x 768 -> 768 int8 6.9 / 7.8. Not taken: 2048 x 768 -> 768 int8 10.1 / 9.6, 8192 x 60 -> 2048 int8 62 / 21,
+// 3639 x 512 -> 150 int16 x int16 19.5 / 13.6.
+struct FewCost {
+    float start, tile, more;
+};
 struct FewCosts {
-    float start[4], tile[4];
-    float other_start, other_tile;
-    float more;
+    FewCost form[4];
+    FewCost whole, stored, ragged;  // the tiled kernels: operands on whole chunks, with results that do not leave from registers, neither
 };
 static constexpr FewCosts FEW_COSTS[] = {
-    /* FEW_I8     */ {{3.9f, 4.1f, 4.0f, 6.8f}, {0.055f, 0.070f, 0.090f, 0.25f}, 6.0f, 0.50f, 0.8f},
-    /* FEW_I16X8  */ {{5.0f, 5.4f, 5.1f, 9.3f}, {0.080f, 0.100f, 0.160f, 0.52f}, 5.2f, 0.82f, 1.1f},
-    /* FEW_I16X16 */ {{5.8f, 6.4f, 6.2f, 0.0f}, {0.120f, 0.140f, 0.270f, 0.00f}, 7.2f, 1.17f, 2.0f},
-    /* FEW_BF16   */ {{3.5f, 3.6f, 3.5f, 5.9f}, {0.050f, 0.060f, 0.100f, 0.25f}, 5.5f, 0.51f, 2.2f},
-    /* FEW_F32    */ {{3.5f, 3.7f, 3.9f, 5.7f}, {0.080f, 0.104f, 0.190f, 0.50f}, 5.5f, 1.80f, 1.1f},
-    /* FEW_FP8    */ {{3.5f, 3.6f, 3.5f, 5.5f}, {0.036f, 0.050f, 0.088f, 0.20f}, 9.7f, 0.46f, 2.4f},
+    /* FEW_I8     */ {{{4.01f, 0.0493f, 0.77f}, {4.24f, 0.0771f, 1.13f}, {4.27f, 0.0955f, 0.95f}, {7.73f, 0.2566f, 2.28f}},
+                      {5.74f, 0.541f, 3.43f}, {7.47f, 0.5496f, 3.76f}, {9.24f, 0.6865f, 4.3f}},
+    /* FEW_I16X8  */ {{{4.84f, 0.0952f, 1.41f}, {6.3f, 0.1333f, 2.46f}, {5.15f, 0.1513f, 2.4f}, {9.52f, 0.3499f, 11.18f}},
+                      {6.5f, 0.7458f, 3.55f}, {6.5f, 0.7458f, 3.55f}, {6.58f, 0.7924f, 5.54f}},
+    /* FEW_I16X16 */ {{{5.7f, 0.0804f, 2.4f}, {6.53f, 0.1623f, 5.57f}, {5.95f, 0.2451f, 5.54f}, {}},
+                      {6.62f, 1.257f, 11.99f}, {6.62f, 1.257f, 11.99f}, {6.58f, 1.238f, 9.0f}},
+    /* FEW_BF16   */ {{{3.37f, 0.0363f, 0.53f}, {3.51f, 0.0589f, 0.65f}, {3.51f, 0.0911f, 0.86f}, {6.06f, 0.1923f, 2.1f}},
+                      {7.22f, 0.5108f, 4.43f}, {7.22f, 0.5108f, 4.43f}, {8.76f, 0.5519f, 4.39f}},
+    /* FEW_F32    */ {{{3.62f, 0.0629f, 0.68f}, {3.89f, 0.1127f, 0.89f}, {4.25f, 0.1843f, 0.93f}, {5.84f, 0.6097f, 2.18f}},
+                      {6.8f, 1.79f, 6.7f}, {6.8f, 1.79f, 6.7f}, {8.37f, 1.788f, 8.77f}},
+    /* FEW_FP8    */ {{{3.66f, 0.0525f, 0.74f}, {3.81f, 0.0651f, 0.83f}, {4.05f, 0.0911f, 1.04f}, {6.75f, 0.1993f, 2.26f}},
+                      {10.67f, 0.4212f, 5.03f}, {10.67f, 0.4212f, 5.03f}, {10.11f, 0.6166f, 5.59f}},
 };
 
+static float launch_us(const FewCost& c, int ktiles, float workgroups) {
+    float per_cu = std::max(1.f, workgroups / 256.f);
+    per_cu = 0.5f * (per_cu + std::ceil(per_cu));  // a last round that is not full overlaps the one before it in part
+    return c.start + c.tile * static_cast<float>(ktiles) * per_cu + c.more * (per_cu - 1.f);
+}
+
+// Reductions of up to 768 on aligned rows have a kernel of their own with little fixed cost (launch_wreg); what is faster here has the
+// weights in fragment order, if they are, and tiles of at most 32 x 32 (those of 64 x 64 are behind launch_wreg at every such size).
+static bool weights_in_registers(const GemmArgs& g, FewKind kind, int batch) { return kind == FEW_I8 && batch == 1 && wreg_applicable(g); }
+
 static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {
-    const FewCosts& c = FEW_COSTS[kind];
     const int ktiles = (g.K + 127) / 128;
     int best = 0;
     *us = 1e30f;
-    for (int f = 0; f < (kind == FEW_I16X16 ? 3 : 4); ++f) {
+    for (int f = 0; f < (kind == FEW_I16X16 || weights_in_registers(g, kind, batch) ? 3 : 4); ++f) {
         const float rows = static_cast<float>((g.M + FEW_FORMS[f].tm * 16 - 1) / (FEW_FORMS[f].tm * 16));
         const float cols = static_cast<float>((g.N + FEW_FORMS[f].tn * 16 - 1) / (FEW_FORMS[f].tn * 16));
-        float per_cu = std::max(1.f, rows * cols * batch / 256.f);
-        if (f == 3) per_cu = std::ceil(per_cu);  // bound by matrix work and L2: a CU with two workgroups takes as long as two
-        const float t = c.start[f] + per_cu * ktiles * c.tile[f] + (per_cu - 1.f) * c.more;
+        const float t = launch_us(FEW_COSTS[kind].form[f], ktiles, rows * cols * static_cast<float>(batch));
         if (t < *us) {
             *us = t;
             best = f;
@@ -492,14 +505,18 @@ bool few_preferred(const GemmArgs& g, FewKind kind, int batch) {
     const bool wide = kind == FEW_I16X8 || kind == FEW_I16X16;
     if (g.K * (wide ? 2 : 1) < 16 || g.M <= 0 || 64 * g.lda >= (int64_t{1} << 31) || 64 * g.ldb >= (int64_t{1} << 31)) return false;
     if (!whole_chunk_rows(g.Bt, g.ldb, g.stride_b, g.K) || (kind == FEW_I16X16 && !whole_chunk_rows(g.Bt_lo, g.ldb, g.stride_b, g.K))) return false;
-    const FewCosts& c = FEW_COSTS[kind];
-    const float tiles = static_cast<float>((g.M + 127) / 128) * static_cast<float>((g.N + 127) / 128) * batch;
-    const int ktiles = (g.K + 127) / 128;
-    float other = (c.other_start + c.other_tile * ktiles) * std::max(1.f, tiles / 256.f);
-    // reductions of up to 768 on aligned rows have a kernel of their own with little fixed cost (launch_wreg)
-    if (kind == FEW_I8 && batch == 1 && wreg_applicable(g)) other = 6.6f + static_cast<float>(g.M) * static_cast<float>(g.N) * static_cast<float>(g.K) * 1.4e-9f;
-    float us;
+    float us, other;
     few_form(g, kind, batch, &us);
+    if (weights_in_registers(g, kind, batch)) {
+        other = 6.6f + static_cast<float>(g.M) * static_cast<float>(g.N) * static_cast<float>(g.K) * 1.4e-9f;
+    } else {
+        const bool whole = g.K * (wide ? 2 : 1) % 16 == 0 && g.lda % 16 == 0 && g.stride_a % 16 == 0 && aligned16(g.A);
+        const float tiles = static_cast<float>((g.M + 127) / 128) * static_cast<float>((g.N + 127) / 128) * static_cast<float>(batch);
+        // (direct_epilogue_ok in gemm.hip)
+        const bool direct = (g.out_kind == A4G_I8 || g.out_kind == A4G_U8) && g.N % 16 == 0 && g.ldc % 16 == 0 && aligned16(g.C);
+        const FewCosts& c = FEW_COSTS[kind];
+        other = launch_us(!whole ? c.ragged : direct ? c.whole : c.stored, (g.K + 127) / 128, tiles);
+    }
     return us < other;
 }
 
