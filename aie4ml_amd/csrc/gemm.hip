@@ -153,17 +153,30 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_i8_nt_kernel(GemmA
         }
     };
 
+    auto load_rows_b = [&](int k0) {
+        if (g.K >= 16) {
+#pragma unroll
+            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load16_any(pb[i] + k0 + min(g.K - (k0 + kb[i]) - 16, 0));
+        } else {
+#pragma unroll
+            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.K);
+        }
+    };
     auto load_tile = [&](int k0) {
         if constexpr (TRANS_A) {
             static_assert(!TRANS_A || RAGGED, "the transposed-A form takes B through the ragged loads");
             load_a_transposed(k0);
-#pragma unroll
-            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.K);
+            load_rows_b(k0);
         } else if constexpr (RAGGED) {
+            // (the branch that load_chunk_ragged has, once for all loads)
+            if (g.K >= 16) {
 #pragma unroll
-            for (int i = 0; i < Cfg::A_PER_T; ++i) ra[i] = load_chunk_ragged(pa[i] + k0, g.K - (k0 + ka[i]), g.K);
+                for (int i = 0; i < Cfg::A_PER_T; ++i) ra[i] = load16_any(pa[i] + k0 + min(g.K - (k0 + ka[i]) - 16, 0));
+            } else {
 #pragma unroll
-            for (int i = 0; i < Cfg::B_PER_T; ++i) rb[i] = load_chunk_ragged(pb[i] + k0, g.K - (k0 + kb[i]), g.K);
+                for (int i = 0; i < Cfg::A_PER_T; ++i) ra[i] = load_chunk_ragged(pa[i] + k0, g.K - (k0 + ka[i]), g.K);
+            }
+            load_rows_b(k0);
         } else {
 #pragma unroll
             for (int i = 0; i < Cfg::A_PER_T; ++i)
@@ -843,9 +856,9 @@ static hipError_t launch_dtl(const GemmArgs& g, int batch, hipStream_t stream) {
 }
 
 // The pipelined kernel takes every K of at least a chunk: 8192 x 17 -> 777 12.4 us, 25.9 on the older tiled one; 8192 x 255 -> 2048
-// 25.6 and 38.3. Only short reductions of hundreds of small problems, where its registers let fewer of them share a CU, stay on
-// that (768 x 100 x 32 x 100: 16.6 us, 17.9 pipelined).
-static bool tiled_is_ahead(const GemmArgs& g, int batch) { return g.K < 16 || (g.K < 160 && batch >= 512); }
+// 25.6 and 38.3. Only hundreds of small problems, where its registers let fewer of them share a CU, stay on that while their reductions are
+// short (768 x 100 x 32 x 100: 16.6 us, 17.9 pipelined; x 197: 22.7 and 24.7; uint8 x 50 30.5 and 33.6, x 160 50.6 and 48.4).
+static bool tiled_is_ahead(const GemmArgs& g, int batch) { return g.K < 16 || (batch >= 512 && g.K < (g.a_unsigned ? 128 : 256)); }
 
 // Picks a kernel and tile shape for the problem. variant: 0 = automatic; 1..4 force a tile shape (tuning only,
 // through the A4G_GEMM_VARIANT environment variable; a forced shape whose kernel's K granularity does not
