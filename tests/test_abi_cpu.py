@@ -117,3 +117,20 @@ def test_argument_validation_happens_before_any_launch(libpath):
     # empty problems are fine and do nothing
     assert lib.a4g_add(None, None, None, 0, 0, 0, 0, None) == 0
     assert lib.a4g_layernorm_i8(None, None, None, None, 0, 64, 1, 7, 5, 6, None) == 0
+
+
+@pytest.mark.parametrize('dim', [16, 32, 48, 64, 80, 96, 112, 128])
+def test_attention_is_long_where_the_other_entry_point_ends(libpath, dim):
+    """ops.attention_is_long names the key counts that a4g_attention_i8 refuses and a4g_attention_long_i8 takes (an empty
+    batch is answered after the checks of the shape, before anything is launched)."""
+    from aie4ml_amd import _lib, ops
+
+    lib = _lib.load()
+
+    def answer(entry, keys):
+        return getattr(lib, entry)(None, None, None, None, 0, 1, 8, keys, dim, None, 6, 0, 0, 23, 0, 0, 0, 15, 0, 7, 0, None)
+
+    for keys in (1, 255, 256, 257, 511, 512, 513, 32768):
+        assert (answer('a4g_attention_i8', keys) != 0) == ops.attention_is_long(dim, keys), keys
+        assert answer('a4g_attention_long_i8', keys) == 0, keys
+    assert answer('a4g_attention_long_i8', 32769) != 0

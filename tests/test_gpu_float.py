@@ -226,3 +226,36 @@ def test_matmul_float_in_place_operand_with_nan_behind_its_rows(ops, fmt, K):
     _lib.check(_lib.load().a4g_matmul_f(ops._ptr(a), ops._float_format(a, 'a'), 0, K, M * K, ops._ptr(b), ld, N * ld, 1, ops._ptr(out), N,
                                         M * N, 1, M, N, K, None, 0, ops._stream()))
     assert torch.equal(out.float().cpu(), torch.from_numpy(A @ B.T))
+
+
+@pytest.mark.parametrize('fmt', FORMATS)
+@pytest.mark.parametrize('M,K,N', [(130, 96, 770), (90, 2000, 1300), (512, 1536, 1024), (300, 1100, 4200), (700, 2000, 2000)])
+def test_dense_float_small_outputs_on_wider_tiles(ops, fmt, M, K, N):
+    """The kernel for small outputs on its tiles of 32 x 16 (the first two sizes), 32 x 32 and 64 x 64 (the last two): K and the output off
+    them. Products of -1, 0 and 1 with at most sixteen that count per row: exact in every format."""
+    r = np.random.default_rng(M + K)
+    t = TORCH_DT[fmt]
+    A, W = np.zeros((M, K), np.float32), r.integers(-1, 2, (K, N)).astype(np.float32)
+    at = r.integers(0, K, (M, 16))
+    A[np.arange(M)[:, None], at] = r.integers(-1, 2, (M, 16))
+    p = ops.pack_dense_float(torch.from_numpy(W).to(t).cuda(), None)
+    got = ops.dense_float(torch.from_numpy(A).to(t).cuda(), p)
+    assert torch.equal(got.float().cpu(), torch.from_numpy(A @ W))
+
+
+@pytest.mark.parametrize('M,N,K', [(8200, 330, 32), (8200, 330, 64), (8200, 330, 129), (8200, 330, 200), (8200, 330, 257), (8200, 330, 512), (8200, 330, 1025),
+                                   (4096, 4096, 512), (4100, 4000, 640)])
+def test_dense_fp8_on_many_tiles(ops, M, N, K):
+    """fp8 with more outputs than the kernel for small ones takes: the tiled kernels of 128 x 128 and (the last two sizes) 256 x 256, K in
+    whole tiles, in whole chunks and off them, rows aligned and at odd bytes between NaN. Exact products as above."""
+    r = np.random.default_rng(M + K)
+    t = torch.float8_e4m3fn
+    A, W = np.zeros((M, K), np.float32), r.integers(-1, 2, (K, N)).astype(np.float32)
+    at = r.integers(0, K, (M, 16))
+    A[np.arange(M)[:, None], at] = r.integers(-1, 2, (M, 16))
+    wide = torch.full((M, K + 3), float('nan')).to(t)
+    wide[:, 1:K + 1] = torch.from_numpy(A).to(t)
+    p = ops.pack_dense_float(torch.from_numpy(W).to(t).cuda(), None)
+    want = torch.from_numpy(A @ W)
+    for x in (torch.from_numpy(A).to(t).cuda(), wide.cuda()[:, 1:K + 1]):
+        assert torch.equal(ops.dense_float(x, p).float().cpu(), want), tuple(x.stride())

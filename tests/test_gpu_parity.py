@@ -638,16 +638,16 @@ def test_matmul_int16_left_operand(ops, oracle, shape, trans_b, b_dtype):
 
 RAGGED = [(300, 200, 100, 0, 0), (257, 130, 1000, 0, 0), (129, 70, 37, 3, 1), (64, 33, 7, 5, 3), (500, 256, 1030, 2, 2),
           (1, 1, 1, 0, 0), (140, 128, 200, 56, 8),
-          # from two K tiles on, rows 4- or 8-byte aligned: descriptor loads by dwords / by 8 bytes, the bytes past K cleared
+          # more than a K tile, on and off the 4- and 8-byte grids
           (300, 144, 1004, 0, 0), (200, 256, 300, 4, 4), (130, 200, 1001, 7, 0), (260, 130, 2042, 6, 8)]
 
 
 @pytest.mark.parametrize('case', RAGGED)
 @pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
 def test_dense_ragged_reduction_and_unaligned_rows(ops, oracle, kind, case):
-    """K that is not a multiple of 16 and activation rows that start at any byte (a column window of a wider matrix)
-    run on the tiled kernels with loads that stop at the row ends: bytes past K must count as zero whatever lies
-    behind them (here: the rest of the wider matrix, filled with extreme values)."""
+    """K that is not a multiple of 16 and activation rows that start at any byte (a column window of a wider matrix): bytes past K
+    must count as zero whatever lies behind them (here: the rest of the wider matrix, filled with extreme values). Outputs as few as
+    these go to the kernel for small ones (K of less than 16 bytes to a tiled one); test_dense_ragged_on_many_tiles has the tiled kernels."""
     M, N, K, extra, off = case
     r = rng(M + N + K + len(kind))
     adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
@@ -1512,3 +1512,62 @@ def test_rows_shorter_than_a_chunk(ops, oracle, K):
         assert np.array_equal(got, oracle.dense(np.ascontiguousarray(X), W, None, np.array([shift]), 'conv_even', out='int16')), (adt, bdt)
     x = gauss8(r, 40, (1000, K))
     assert np.array_equal(host(ops.softmax_exp(dev(x), 23)), oracle.softmax_exp(x, 23))
+
+
+@pytest.mark.parametrize('K,extra,off', [(300, 4, 4), (1000, 0, 0), (1001, 7, 0), (1004, 0, 0), (1030, 2, 2), (2042, 6, 8)])
+@pytest.mark.parametrize('kind', ['int8', 'uint8', 'int16x8', 'int16x16'])
+def test_dense_ragged_on_many_tiles(ops, oracle, kind, K, extra, off):
+    """The same windows with more outputs than the kernel for small ones takes: the tiled kernels, with K of several tiles on
+    and off the 4-, 8- and 16-byte grids, partial last tiles of rows and columns."""
+    r = rng(K + len(kind))
+    M, N = 8200, 330
+    adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
+    info = np.iinfo(adt)
+    wide = np.full((M, off + K + extra), info.max, dtype=adt)
+    wide[:, off + K:] = info.min
+    A = wide[:, off:off + K] = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+    W = r.integers(-32768, 32768, (K, N)).astype(np.int16) if kind == 'int16x16' else gauss8(r, 40, (K, N))
+    bias = r.integers(-2**15, 2**15, N).astype(np.int32)
+    top = 28 if kind == 'int16x16' else (18 if kind == 'int16x8' else 12)
+    shifts = r.integers(top - 5, top + 1, N).astype(np.int32)
+    p = ops.pack_dense(dev(W), dev(bias), shifts)
+    want = oracle.dense(np.ascontiguousarray(A), W, bias, shifts, 'conv_even', relu=True, out='int8')
+    assert np.array_equal(host(ops.dense(dev(wide)[:, off:off + K], p, 'conv_even', relu=True, out_kind='int8')), want)
+
+
+@pytest.mark.parametrize('M,N,K', [(1, 16, 16), (40, 48, 144), (100, 272, 768), (300, 272, 400), (1500, 48, 272), (300, 528, 640), (700, 272, 128),
+                                   (333, 528, 48)])
+@pytest.mark.parametrize('a_dtype', [np.int8, np.uint8])
+def test_small_outputs_on_weights_in_fragment_order(ops, oracle, a_dtype, M, N, K):
+    """Reductions of up to 768 whose weights lie in fragment order, too: tiles of 16 x 16 (the first three sizes), 32 x 16 (two) and
+    32 x 32 (three); column counts off the groups of 32 in which that order mixes them, K on and off a K tile, shifts that the
+    other kernel for such reductions takes, both one-byte results."""
+    if a_dtype == np.uint8 and K > 640:
+        K = 640  # unsigned activations: see wreg_applicable
+    r = rng(M + N + K)
+    info = np.iinfo(a_dtype)
+    A = r.integers(info.min, info.max + 1, (M, K)).astype(a_dtype)
+    W = gauss8(r, 40, (K, N))
+    bias = r.integers(-2**14, 2**14, N).astype(np.int32)
+    for shifts in (np.array([9], np.int32), r.integers(1, 16, N).astype(np.int32)):
+        p = ops.pack_dense(dev(W), dev(bias), shifts if len(shifts) > 1 else int(shifts[0]))
+        assert p.wf is not None
+        for mode, relu, out in (('conv_even', True, 'int8'), ('symmetric_inf', False, 'uint8'), ('floor', False, 'int8')):
+            got = host(ops.dense(dev(A), p, mode, relu=relu, out_kind=out))
+            assert np.array_equal(got, oracle.dense(A, W, bias, shifts, mode, relu=relu, out=out)), (mode, out)
+
+
+@pytest.mark.parametrize('kind,M,N,K', [('int8', 130, 770, 1000), ('uint8', 64, 1100, 3000), ('int8', 200, 2000, 2000), ('int16x8', 512, 2048, 1500),
+                                        ('int16x16', 130, 770, 1000), ('int16x16', 200, 2000, 700), ('int8', 600, 2000, 1500)])
+def test_small_outputs_on_wider_tiles(ops, oracle, kind, M, N, K):
+    """The kernel for small outputs on its tiles of 32 x 16 and up, rows, columns and K off them; accumulators that wrap."""
+    r = rng(M + N + K)
+    adt = {'int8': np.int8, 'uint8': np.uint8}.get(kind, np.int16)
+    info = np.iinfo(adt)
+    A = r.integers(info.min, info.max + 1, (M, K)).astype(adt)
+    W = r.integers(-32768, 32768, (K, N)).astype(np.int16) if kind == 'int16x16' else gauss8(r, 40, (K, N))
+    bias = r.integers(-2**31, 2**31, N).astype(np.int32)
+    shift = 28 if kind == 'int16x16' else 18 if kind == 'int16x8' else 11
+    p = ops.pack_dense(dev(W), dev(bias), shift)
+    got = host(ops.dense(dev(A), p, 'conv_even', out_kind='int16'))
+    assert np.array_equal(got, oracle.dense(A, W, bias, np.array([shift]), 'conv_even', out='int16'))
