@@ -360,16 +360,21 @@ class GPUModel:
             attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode,
                    out=heads_view(out, 0))
             values[grp['out']] = out
-        elif not _attention_launch_takes(values[tr0['q']], values[tr0['k']], values[tr0['v']]):
+            return
+        q, k, v = values[tr0['q']], values[tr0['k']], values[tr0['v']]
+        d, keys = int(q.shape[-1]), int(k.shape[-2])
+        long = ops.attention_is_long(d, keys)
+        if not _attention_launch_takes(q, k, v) or \
+                (long and not ops.attention_long_pays(q.numel() // max(1, d * int(q.shape[-2])), int(q.shape[-2]), keys, d)):
             self._run_attention_unfused(grp, values)
-        else:
-            q, k, v = values[tr0['q']], values[tr0['k']], values[tr0['v']]
-            attend = ops.attention_long if ops.attention_is_long(int(q.shape[-1]), int(k.shape[-2])) else ops.attention
-            values[grp['out']] = attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode)
+            return
+        attend = ops.attention_long if long else ops.attention
+        values[grp['out']] = attend(q, k, v, c1.shift, c1.rounding_mode, sm, c3.shift, c3.rounding_mode)
 
     def _run_attention_unfused(self, grp, values, heads_view=None) -> None:
         """The members of a planned attention group one operator at a time: MatMul, Softmax, MatMul per head, then the
-        concat. Taken when the operands turn out at run time to lie as the fused launch does not take them."""
+        concat. Taken when the operands turn out at run time to lie as the fused launch does not take them, or to be so
+        few that it would leave the chip idle."""
         execution, graph = self.context.ir.execution, self.context.ir.logical
         for h, tr in enumerate(grp['heads']):
             if heads_view is not None:  # head h of the [batch, heads, seq, d] views, should its slice node come later

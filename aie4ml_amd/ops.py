@@ -635,6 +635,21 @@ def attention_is_long(head_dim: int, keys: int) -> bool:
     return keys > (256 if head_dim > 64 else 512)
 
 
+def attention_long_pays(problems: int, queries: int, keys: int, head_dim: int) -> bool:
+    """Whether attention_long() is ahead of batched matmul(), Softmax and matmul() on that many problems. A workgroup takes all the keys of
+    its rows, so that few rows leave the chip idle; the wide heads, at four matrix instructions a step, lose by that. Measured, this / three
+    launches, us: head dimension 128, one problem of 1024 x 1024 96 / 58, of 1 x 4096 356 / 138, of 128 x 16384 1404 / 1025, 16 of 1024 x
+    1024 97 / 101, one of 1 x 300 34 / 32; dimension 96, one of 128 x 4096 201 / 141, of 128 x 600 38 / 43, of 128 x 16384 782 / 1030;
+    dimension 64, one of 1 x 4096 110 / 132, of 1024 x 1024 33 / 53 (32: 29 / 22, where the host takes longer than either)."""
+    if head_dim <= 64:
+        return True
+    few = 16 if head_dim <= 96 else 32 if keys < 1500 else 64
+    if problems * ((queries + 255) // 256) > few:
+        return True
+    alone = 9.0 + (0.0472 if head_dim <= 96 else 0.0855) * keys
+    return 24.0 + 0.031 * min(keys, 4096) + 0.073 * max(keys - 4096, 0) >= 0.9 * alone
+
+
 def attention_long(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logit_shift: int, logit_rounding, softmax: dict,
                    out_shift: int, out_rounding, out: Optional[torch.Tensor] = None):
     """attention() for any number of keys up to 32768 (same arguments, same integers, one launch): the kernel walks the keys

@@ -710,3 +710,19 @@ def test_head_slices_made_on_demand(oracle, case, seq):
     assert grp['concat'] and len(grp['heads']) == heads
     xin = np.clip(np.rint(r.normal(0, 24, (batch, seq, pad + 3 * heads * d))), -128, 127).astype(np.int8)
     _graph_check(model, oracle, {'x': xin})
+
+
+@pytest.mark.parametrize('lead,sq,sk,d,fused', [((1,), 40, 600, 128, False), ((70,), 5, 600, 128, True), ((1,), 40, 300, 128, True), ((2,), 3, 2050, 96, False),
+                                                ((2,), 3, 600, 96, True), ((1,), 9, 2050, 64, True)])
+def test_few_wide_heads_with_many_keys_run_operator_by_operator(oracle, lead, sq, sk, d, fused):
+    """A lone triple whose rows fill a few workgroups of the long attention kernel only: three launches where those are ahead."""
+    import torch
+
+    r = np.random.default_rng(sk + d)
+    model = _triple(lead, sq, sk, d)
+    x = {n: np.clip(np.rint(r.normal(0, 24, lead + (s, d))), -128, 127).astype(np.int8) for n, s in (('q', sq), ('k', sk), ('v', sk))}
+    _graph_check(model, oracle, x)
+    seen = []
+    model._run_attention_unfused = lambda grp, values: seen.append(1) or type(model)._run_attention_unfused(model, grp, values)
+    model.execute({n: torch.from_numpy(a).cuda() for n, a in x.items()})
+    assert (not seen) is fused
