@@ -426,20 +426,16 @@ def _attention_launch_takes(q, k, v) -> bool:
     points ask for contiguous int8 rows on 16-byte aligned addresses, row pitches of at least a row, keys (and, for the
     long one, values) of a head within 2 GiB, and a number of query rows that their grid can count. Shapes, shifts
     and Softmax parameters are the planner's to check: they are known when the graph is compiled."""
-    rows, keys, dim = int(q.shape[-2]), int(k.shape[-2]), int(q.shape[-1])
-    for t in (q, k, v):
-        stride = t.stride()
-        if stride[-1] != 1 or stride[-2] < dim:
-            return False
-        at = t.data_ptr()
-        for st in stride[:-1]:
-            at |= st  # (a power of two divides all of them if it divides their bitwise or)
-        if at % 16:
-            return False
-    blocks = (rows + 127) // 128
-    for extent in q.shape[:-2]:
-        blocks *= int(extent)
-    return (keys + 32) * max(k.stride(-2), v.stride(-2)) < 1 << 31 and rows <= 1 << 24 and blocks < 1 << 31
+    sq, sk, sv = q.stride(), k.stride(), v.stride()
+    rows, dim = q.size(-2), q.size(-1)
+    if sq[-1] * sk[-1] * sv[-1] != 1 or sq[-2] < dim or sk[-2] < dim or sv[-2] < dim:
+        return False
+    at = q.data_ptr() | k.data_ptr() | v.data_ptr()
+    for st in sq[:-1] + sk[:-1] + sv[:-1]:
+        at |= st  # (a power of two divides all of them if it divides their bitwise or)
+    if at % 16 or (k.size(-2) + 32) * max(sk[-2], sv[-2]) >= 1 << 31 or rows > 1 << 24:
+        return False
+    return q.numel() < dim << 31 or q.numel() // (dim * rows) * ((rows + 127) // 128) < 1 << 31
 
 
 def _mlp_layers_are_faster(rows: int, layers, on_matrix_units: bool = False) -> bool:
