@@ -5,12 +5,13 @@
 // rows three times and keeps nothing per key: (1) the row maximum, taken on the raw accumulators (rounding and saturation
 // are monotone, so one rounding per row is enough: half a vector instruction per logit), (2) the sum of the scores,
 // (3) the probabilities, which go straight into the second matrix product. The logits of (2) and (3) are formed again:
-// two matrix instructions and two vector instructions per logit cost less than what storing them would: 1024 keys of
-// 128 rows are 128 KiB, which leaves one wave per SIMD, and a lone wave issues vector instructions at half the rate of two.
-// Bound by vector issue and by the latencies between its steps (9-10 instructions per logit). Two workgroups of four waves
+// two products of 32 x 32 logits more (two matrix instructions each at dimension 64) and about two vector instructions per logit
+// cost less than what storing them would: 1024 keys of 128 rows are 128 KiB, which leaves one wave per SIMD, and a lone wave issues
+// vector instructions at half the rate of two.
+// Bound by vector issue and by the latencies between its steps (12 vector instructions per logit in all, by the counter). Two workgroups of four waves
 // share a CU; the score table is stored once per LDS bank (a single copy would serialise the gathers: two per logit).
-// Measured (head dimension 64, as many queries as keys): 48 heads of 1024 keys 42.6 us, 192 heads 114 us (18 ns per 1000
-// logits of a head against 9.7 in attention_kernel at 512 keys); MatMul, Softmax and MatMul head by head through memory
+// Measured (head dimension 64, as many queries as keys): 48 heads of 1024 keys 42.6 us, 192 heads 114 us (0.57 ns per 1000
+// logits with the chip full, 0.36 in attention_kernel at 512 keys); MatMul, Softmax and MatMul head by head through memory
 // took more than 1000 us for the 48 heads. By walks, of the 192 heads' time: 13 / 26 / 54 us, the rest is each workgroup's
 // start and end. Scores gathered a tile ahead of their use: no gain (112 us), and four waves per SIMD do not fit the
 // registers (128 a lane: 190 us with the spills).

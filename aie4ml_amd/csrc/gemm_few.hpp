@@ -1,4 +1,4 @@
-// Dense and MatMul with too few output tiles to fill the chip with the tiled kernels (gemm_few.hip).
+// Dense, and float MatMul, with too few output tiles to fill the chip with the tiled kernels (gemm_few.hip).
 #pragma once
 
 #include "gemm_rs.hpp"
