@@ -177,9 +177,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(GemmArgs g, int tiles
     };
     v4i fa[TM][NA], fb[PLANES][TN][2];  // fragments of the tile in hand
     // Registers of a tile -> the wave's patch -> fragments, in blocks of sixteen rows. The 64 x 64 tiles have one K tile on its way: a
-    // block is read back as soon as its rows have arrived (447 x 4736 -> 2295 fp8 15.6 us, 17.6 with all writes ahead of all reads); the
-    // others have several, and registers to save.
-    constexpr bool BLOCKS = TM == 4;
+    // block is read back as soon as its rows have arrived (447 x 4736 -> 2295 fp8 15.6 us, 17.6 with all writes ahead of all reads). So do
+    // bfloat16 and float32 (200 sizes each 1.5 and 0.8 % faster); int8 on 32 x 32 tiles would lose its fourth wave per SIMD to it (20 %).
+    constexpr bool BLOCKS = TM == 4 || KIND == FEW_BF16 || KIND == FEW_F32;
     auto put_a = [&](int slot, int i) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = i * (LA / TM); t < (i + 1) * (LA / TM); ++t) {
@@ -447,10 +447,10 @@ static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStr
 }
 
 // What a launch takes, in us: `start`, plus `tile` for every K tile of 128 bytes and every workgroup that a CU gets (at least one), plus
-// `more` for every workgroup of a CU after its first. The tiled kernels by the same law with their 128 x 128 tiles. Fitted to 800 random
-// sizes in every format (2400 in int8) at which every form and the tiled kernel were timed: 1 to 16384 rows, 32 to 8192 inputs, 8 to
+// `more` for every workgroup of a CU after its first. The tiled kernels by the same law with their 128 x 128 tiles. Fitted to 1400 random
+// sizes in every format (4200 in int8) at which every form and the tiled kernel were timed: 1 to 16384 rows, 32 to 8192 inputs, 8 to
 // 8192 outputs, from a workgroup in all to hundreds for a CU; where the law is coarse the constants are the ones that pick best.
-// What is picked is within 0.1 % of the fastest on average (int8 and int16 0.2 %, float32 0.7 %). Measured, this kernel / the tiled ones, us:
+// What is picked is within 0.1 % of the fastest on average at 600 other sizes a format (int8 0.3 %, bfloat16 and int16 0.5 %, float32 0.8 %). Measured, this kernel / the tiled ones, us:
 // 16 x 4096 -> 4096 int8 5.4 / 22.3, int16 7.5 / 51, bfloat16 6.7 / 38, float32 14 / 235, fp8 4.6 / 24; 128 x 768 -> 768 int8
 // 4.6 / 7.7; 1024 x 768 -> 768 int8 6.9 / 7.8. Not taken: 2048 x 768 -> 768 int8 10.1 / 9.6, 8192 x 60 -> 2048 int8 62 / 21,
 // 3639 x 512 -> 150 int16 x int16 19.5 / 13.6.
@@ -462,18 +462,18 @@ struct FewCosts {
     FewCost whole, stored, ragged;  // the tiled kernels: operands on whole chunks, with results that do not leave from registers, neither
 };
 static constexpr FewCosts FEW_COSTS[] = {
-    /* FEW_I8     */ {{{4.01f, 0.0493f, 0.77f}, {4.24f, 0.0771f, 1.13f}, {4.27f, 0.0955f, 0.95f}, {7.73f, 0.2566f, 2.28f}},
-                      {5.74f, 0.541f, 3.43f}, {7.47f, 0.5496f, 3.76f}, {9.24f, 0.6865f, 4.3f}},
-    /* FEW_I16X8  */ {{{4.84f, 0.0952f, 1.41f}, {6.3f, 0.1333f, 2.46f}, {5.15f, 0.1513f, 2.4f}, {9.52f, 0.3499f, 11.18f}},
-                      {6.5f, 0.7458f, 3.55f}, {6.5f, 0.7458f, 3.55f}, {6.58f, 0.7924f, 5.54f}},
-    /* FEW_I16X16 */ {{{5.7f, 0.0804f, 2.4f}, {6.53f, 0.1623f, 5.57f}, {5.95f, 0.2451f, 5.54f}, {}},
-                      {6.62f, 1.257f, 11.99f}, {6.62f, 1.257f, 11.99f}, {6.58f, 1.238f, 9.0f}},
-    /* FEW_BF16   */ {{{3.37f, 0.0363f, 0.53f}, {3.51f, 0.0589f, 0.65f}, {3.51f, 0.0911f, 0.86f}, {6.06f, 0.1923f, 2.1f}},
-                      {7.22f, 0.5108f, 4.43f}, {7.22f, 0.5108f, 4.43f}, {8.76f, 0.5519f, 4.39f}},
-    /* FEW_F32    */ {{{3.62f, 0.0629f, 0.68f}, {3.89f, 0.1127f, 0.89f}, {4.25f, 0.1843f, 0.93f}, {5.84f, 0.6097f, 2.18f}},
-                      {6.8f, 1.79f, 6.7f}, {6.8f, 1.79f, 6.7f}, {8.37f, 1.788f, 8.77f}},
-    /* FEW_FP8    */ {{{3.66f, 0.0525f, 0.74f}, {3.81f, 0.0651f, 0.83f}, {4.05f, 0.0911f, 1.04f}, {6.75f, 0.1993f, 2.26f}},
-                      {10.67f, 0.4212f, 5.03f}, {10.67f, 0.4212f, 5.03f}, {10.11f, 0.6166f, 5.59f}},
+    /* FEW_I8     */ {{{4.05f, 0.0472f, 0.65f}, {4.53f, 0.0558f, 1.14f}, {4.26f, 0.0892f, 0.81f}, {7.92f, 0.2474f, 1.31f}},
+                      {5.43f, 0.5193f, 3.54f}, {6.68f, 0.5456f, 3.98f}, {8.82f, 0.6466f, 4.35f}},
+    /* FEW_I16X8  */ {{{4.97f, 0.076f, 1.28f}, {5.92f, 0.1001f, 4.11f}, {4.97f, 0.1958f, 2.19f}, {10.26f, 0.3652f, 11.32f}},
+                      {5.63f, 0.7455f, 3.83f}, {5.63f, 0.7455f, 3.83f}, {6.16f, 0.8082f, 5.64f}},
+    /* FEW_I16X16 */ {{{5.68f, 0.0917f, 2.23f}, {6.52f, 0.1483f, 5.98f}, {5.8f, 0.2706f, 5.62f}, {}},
+                      {6.55f, 1.297f, 12.71f}, {6.55f, 1.297f, 12.71f}, {6.28f, 1.344f, 10.37f}},
+    /* FEW_BF16   */ {{{3.52f, 0.0509f, 0.7f}, {3.53f, 0.0705f, 0.74f}, {3.78f, 0.0864f, 0.88f}, {5.99f, 0.1925f, 2.94f}},
+                      {8.0f, 0.5162f, 4.42f}, {8.0f, 0.5162f, 4.42f}, {10.36f, 0.5061f, 3.54f}},
+    /* FEW_F32    */ {{{3.62f, 0.0654f, 0.9f}, {3.9f, 0.1175f, 0.84f}, {4.33f, 0.1585f, 1.05f}, {5.8f, 0.6075f, 2.47f}},
+                      {7.17f, 1.886f, 6.34f}, {7.17f, 1.886f, 6.34f}, {7.5f, 1.901f, 8.99f}},
+    /* FEW_FP8    */ {{{3.68f, 0.039f, 0.8f}, {3.8f, 0.0697f, 0.97f}, {3.9f, 0.0913f, 1.11f}, {6.68f, 0.2032f, 2.64f}},
+                      {10.56f, 0.4347f, 5.38f}, {10.56f, 0.4347f, 5.38f}, {10.99f, 0.6238f, 5.57f}},
 };
 
 static float launch_us(const FewCost& c, int ktiles, float workgroups) {
