@@ -429,11 +429,8 @@ template <int KIND>
 static hipError_t launch_few_kind(const GemmArgs& g, int batch, int form, hipStream_t stream) {
     if constexpr (KIND == FEW_I8) {
         if (g.Wf && batch == 1 && aligned16(g.Wf) && wreg_applicable(g) && rowpacked_bytes(g.N, g.K) < (int64_t{1} << 31)) {
-            switch (form) {
-            case 0: return launch_few_tile<KIND, 4, 1, 1, 4, true>(g, batch, stream);
-            case 1: return launch_few_tile<KIND, 4, 2, 1, 3, true>(g, batch, stream);
-            default: return launch_few_tile<KIND, 4, 2, 2, 2, true>(g, batch, stream);
-            }
+            // (no size picks 32 x 16)
+            return form == 0 ? launch_few_tile<KIND, 4, 1, 1, 4, true>(g, batch, stream) : launch_few_tile<KIND, 4, 2, 2, 2, true>(g, batch, stream);
         }
     }
     switch (form) {
@@ -483,7 +480,7 @@ static float launch_us(const FewCost& c, int ktiles, float workgroups) {
 }
 
 // Reductions of up to 768 on aligned rows have a kernel of their own with little fixed cost (launch_wreg); what is faster here has the
-// weights in fragment order, if they are, and tiles of at most 32 x 32 (those of 64 x 64 are behind launch_wreg at every such size).
+// weights in fragment order, if they are, and tiles of 16 x 16 or 32 x 32 (those of 64 x 64 are behind launch_wreg at every such size).
 static bool weights_in_registers(const GemmArgs& g, FewKind kind, int batch) { return kind == FEW_I8 && batch == 1 && wreg_applicable(g); }
 
 static int few_form(const GemmArgs& g, FewKind kind, int batch, float* us) {

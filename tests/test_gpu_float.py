@@ -229,10 +229,10 @@ def test_matmul_float_in_place_operand_with_nan_behind_its_rows(ops, fmt, K):
 
 
 @pytest.mark.parametrize('fmt', FORMATS)
-@pytest.mark.parametrize('M,K,N', [(130, 96, 770), (90, 2000, 1300), (512, 1536, 1024), (300, 1100, 4200), (700, 2000, 2000)])
+@pytest.mark.parametrize('M,K,N', [(130, 96, 770), (90, 2000, 1300), (512, 1536, 1024), (300, 1100, 4200), (700, 2000, 2000), (300, 200, 3000)])
 def test_dense_float_small_outputs_on_wider_tiles(ops, fmt, M, K, N):
-    """The kernel for small outputs on its tiles of 32 x 16 (the first two sizes), 32 x 32 and 64 x 64 (the last two): K and the output off
-    them. Products of -1, 0 and 1 with at most sixteen that count per row: exact in every format."""
+    """The kernel for small outputs on its tiles of 32 x 16 (the first two sizes), 32 x 32 and 64 x 64 (the last three; float32 the
+    last one): K and the output off them. Products of -1, 0 and 1 with at most sixteen that count per row: exact in every format."""
     r = np.random.default_rng(M + K)
     t = TORCH_DT[fmt]
     A, W = np.zeros((M, K), np.float32), r.integers(-1, 2, (K, N)).astype(np.float32)

@@ -1539,8 +1539,8 @@ def test_dense_ragged_on_many_tiles(ops, oracle, kind, K, extra, off):
                                    (333, 528, 48)])
 @pytest.mark.parametrize('a_dtype', [np.int8, np.uint8])
 def test_small_outputs_on_weights_in_fragment_order(ops, oracle, a_dtype, M, N, K):
-    """Reductions of up to 768 whose weights lie in fragment order, too: tiles of 16 x 16 (the first three sizes), 32 x 16 (two) and
-    32 x 32 (three); column counts off the groups of 32 in which that order mixes them, K on and off a K tile, shifts that the
+    """Reductions of up to 768 whose weights lie in fragment order, too: tiles of 16 x 16 (the first three sizes) and of 32 x 32 (the
+    others); column counts off the groups of 32 in which that order mixes them, K on and off a K tile, shifts that the
     other kernel for such reductions takes, both one-byte results."""
     if a_dtype == np.uint8 and K > 640:
         K = 640  # unsigned activations: see wreg_applicable
